@@ -557,6 +557,7 @@ struct hm_system
         k.counter = st;
         k.check_delay = check_delay;
         k.dist_check = dist_check;
+        k.slot_of = slot_of;
         if (uses_rel())
         {
             // the cell ordering of this build wrote the relative positions the list stages
@@ -1035,6 +1036,12 @@ struct hm_system
         nl_log.clear();
         if (rcut_max <= 0.0 || !nlist)
             return;
+        {
+            NlistKernelArgs k;
+            fill_nlist_args(k, false);
+            if (nlist_uses_columns(k))
+                return;  // one launch shape
+        }
         std::vector<int> shapes{0};
         if (cmax <= 64)
             shapes = {NL_SHAPE_TINY, NL_SHAPE_SMALL, NL_SHAPE_MID, NL_SHAPE_BIG};

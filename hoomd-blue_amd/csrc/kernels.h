@@ -195,6 +195,7 @@ struct NlistKernelArgs
     const float3* srel;
     const unsigned int* sidx;
     const uint32_t* swrd;
+    const uint32_t* slot_of;  // slot of each particle (exclusions of rows with offset codes)
     float cwf[3];             // cell widths rounded to FP32
     // launch shape, 0 = chosen from the cell occupancy. shape: workgroup form of the FP32 path
     // (NL_SHAPE_*; a form whose home-cell capacity is below cmax falls back to the default);
@@ -263,6 +264,8 @@ hipError_t launch_cell_bin_rank(unsigned int N, const unsigned int dim[3], unsig
                                 const StepState* gate, hipStream_t s, const DevBox& box,
                                 const RelFrame& rel);
 hipError_t launch_nlist_build(const NlistKernelArgs& a, hipStream_t s);
+// whether that launch builds over columns of cells (its shape and grid are then not used)
+bool nlist_uses_columns(const NlistKernelArgs& a);
 
 hipError_t launch_nlist_check(unsigned int N, const double4* pos, const d3* last,
                               const DevBox& box, double maxsq, unsigned int* flag, hipStream_t s);

@@ -7,7 +7,9 @@
 #include <type_traits>
 
 #include "evaluators.h"
+#include "kernel_util.h"
 #include "kernels.h"
+#include "tile.h"
 
 namespace hm
 {
@@ -64,35 +66,6 @@ hipError_t launch_cell_adj(const unsigned int dim[3], unsigned int* adj, hipStre
     hipLaunchKernelGGL(cell_adj_kernel, dim3((ncell + 255) / 256), dim3(256), 0, s, dim[0],
                        dim[1], dim[2], n_adj, adj);
     return hipGetLastError();
-}
-
-// ======================================================================== persistent grids
-// Kernels that only run on a neighbour-list rebuild are launched every step and exit at once
-// when the device-side rebuild flag is not set. They walk their work in grid-stride loops over a
-// bounded grid, so an idle step costs a few hundred empty workgroups instead of one per cell.
-constexpr unsigned int GATED_BLOCKS = 2048;
-
-__device__ __forceinline__ bool gate_closed(const StepState* gate)
-{
-    return gate && gate->rebuild_at != gate->timestep + 1;
-}
-
-// XCD-aware persistent loop: workgroup b runs on XCD (b % 8); it visits the items of that XCD's
-// contiguous eighth of [0, n) with stride gridDim.x / 8.
-struct XcdRange
-{
-    unsigned int begin, end, stride;
-};
-
-__device__ __forceinline__ XcdRange xcd_range(unsigned int n)
-{
-    const unsigned int xcd = blockIdx.x & 7u, r = blockIdx.x >> 3, per = gridDim.x >> 3;
-    const unsigned int chunk = (n + 7) / 8;
-    XcdRange x;
-    x.begin = xcd * chunk + r;
-    x.end = min(n, (xcd + 1) * chunk);
-    x.stride = per;
-    return x;
 }
 
 // ======================================================================== cell build
@@ -456,8 +429,9 @@ __device__ __forceinline__ void rank_particle(unsigned int i, unsigned int cmax,
             rf.rel[slot] = make_float3(rr.x, rr.y, rr.z);
             rf.relw[slot] = pc;
             const_cast<uint32_t*>(rf.pcell)[i] = pc;
-            const_cast<uint32_t*>(rf.slot_of)[i] = slot;
         }
+        if (rf.slot_of)
+            const_cast<uint32_t*>(rf.slot_of)[i] = slot;
     }
 }
 
@@ -601,41 +575,6 @@ __device__ __forceinline__ void pass_bounds(unsigned int n_adj, const unsigned i
     }
 }
 
-__device__ __forceinline__ void load_exclusions(const NlistKernelArgs& a, unsigned int i,
-                                                unsigned int& ex0, unsigned int& ex1,
-                                                unsigned int& ex2, unsigned int& ex3)
-{
-    unsigned int ne = min(a.n_excl[i], a.max_excl);
-    const unsigned int* er = a.excl + (size_t)i * a.max_excl;
-    if (ne > 0)
-        ex0 = er[0];
-    if (ne > 1)
-        ex1 = er[1];
-    if (ne > 2)
-        ex2 = er[2];
-    if (ne > 3)
-        ex3 = er[3];
-}
-
-// The k-th smallest (k = 0, 1, 2) of the wrapped coordinates h - 1, h, h + 1 on an axis of
-// d >= 3 cells; returns its offset from h and sets n to the coordinate.
-__device__ __forceinline__ int sorted_neighbour(int h, int d, int k, int& n)
-{
-    int off;
-    if (h == 0)  // h - 1 wraps to d - 1, the largest
-        off = k == 0 ? 0 : (k == 1 ? 1 : -1);
-    else if (h == d - 1)  // h + 1 wraps to 0, the smallest
-        off = k == 0 ? 1 : (k == 1 ? -1 : 0);
-    else
-        off = k - 1;
-    n = h + off;
-    if (n < 0)
-        n += d;
-    else if (n >= d)
-        n -= d;
-    return off;
-}
-
 // load_exclusions without the count-to-row dependency: the row's first four entries (within the
 // row's max_excl) are read together with the count, then masked by it
 __device__ __forceinline__ void load_exclusions_flat(const NlistKernelArgs& a, unsigned int i,
@@ -658,17 +597,6 @@ __device__ __forceinline__ void load_exclusions_flat(const NlistKernelArgs& a, u
     ex1 = ne > 1 ? v1 : 0xffffffffu;
     ex2 = ne > 2 ? v2 : 0xffffffffu;
     ex3 = ne > 3 ? v3 : 0xffffffffu;
-}
-
-// Minimum-image offset of a position from a cell centre, rounded to FP32 (dims >= 4 keeps every
-// staged particle within 1.5 cell widths of the centre, well inside half a box).
-__device__ __forceinline__ float3 rel_to_centre(const DevBox& b, double x, double y, double z,
-                                                double cx, double cy, double cz)
-{
-#pragma clang fp contract(off)
-    double dx = x - cx, dy = y - cy, dz = z - cz;
-    min_image(b, dx, dy, dz);
-    return make_float3((float)dx, (float)dy, (float)dz);
 }
 
 __device__ __forceinline__ void cell_centre(const DevBox& b, const unsigned int* dim,
@@ -1041,21 +969,7 @@ void nlist_kernel(NlistKernelArgs a)
     __shared__ NlistShared<FAST, MT, EXCL, C> S;
     if (gate_closed(a.gate))
         return;
-    if (a.counter && blockIdx.x == 0 && threadIdx.x == 0)
-    {
-        // build statistics of NeighborList::needsUpdating (NeighborList.cc:1349-1415)
-        StepState* st = a.counter;
-        const unsigned long long t1 = st->timestep + 1;
-        if (st->forced_at != t1)
-        {
-            if (t1 > st->last_update && t1 - st->last_update < st->shortest)
-                st->shortest = t1 - st->last_update;
-            if (a.dist_check && a.check_delay > 1 && t1 == st->last_update + a.check_delay)
-                st->n_dangerous++;
-        }
-        st->last_update = t1;
-        st->n_builds++;
-    }
+    count_build(a);
     const XcdRange r = xcd_range(a.ncell);
     for (unsigned int cell = r.begin; cell < r.end; cell += r.stride)
         nlist_cell<FAST, MT, EXCL, C>(a, cell, S);
@@ -1076,10 +990,34 @@ static void nlist_dispatch(const NlistKernelArgs& a, bool mt, bool ex, unsigned 
                            a);
 }
 
+// Cells of a few particles are built over columns (tile.hip). Index rows, us a build, cell form below ->
+// columns: 10^6 particles, 3.0 a cell 405 -> 254, 6.7 a cell 397 -> 302; 131 072, 3.1 a cell 58 -> 38,
+// 7.5 a cell 59 -> 43; 50 021, 3.2 a cell 27 -> 22, 7.3 a cell 28 -> 24; at 16 384 the two are equal
+// (15 -> 16), and at 21 a cell the cell form's wavefront per home particle is the better one (520
+// against 606 at 10^6). The cell form also keeps the 16-bit local rows, grids with fewer than 4
+// cells along an axis, and exclusions given without the slot of each particle.
+constexpr unsigned int COL_MIN_N = 32768;
+
+static bool column_build_applies(const NlistKernelArgs& a, ColGeom& g)
+{
+    return a.pos && (a.entries || a.srel) && !a.lrow && !a.skip_index_rows && a.n_adj == 27
+           && (!a.offset_codes || a.sidx) && (!a.n_excl || a.max_excl == 0 || a.slot_of)
+           && a.N >= COL_MIN_N && a.N <= 8ull * a.ncell && choose_columns(a.N, a.dim, g);
+}
+
+bool nlist_uses_columns(const NlistKernelArgs& a)
+{
+    ColGeom g;
+    return column_build_applies(a, g);
+}
+
 hipError_t launch_nlist_build(const NlistKernelArgs& a_in, hipStream_t s)
 {
     if (a_in.ncell == 0)
         return hipSuccess;
+    ColGeom cg;
+    if (column_build_applies(a_in, cg))
+        return launch_nlist_columns(a_in, cg, s);
     NlistKernelArgs a = a_in;
     const unsigned int grid = round_up(a.grid ? a.grid : min(a.ncell, GATED_BLOCKS), 8);
     // small cells: a few particles per cell on average, and every home cell fits the
