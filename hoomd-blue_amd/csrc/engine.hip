@@ -199,6 +199,8 @@ struct hm_system
     StepState* h_st = nullptr;
     Conditions* h_cond = nullptr;
     double* ke_partial = nullptr;
+    BussiDraws* draws = nullptr;
+    unsigned int n_draws = 0;
     unsigned int n_partial = 0;
     double* thermo_partial = nullptr;
     double* thermo_out = nullptr;
@@ -337,6 +339,7 @@ struct hm_system
         h_cond = nullptr;
         h_thermo = nullptr;
         dfree(ke_partial);
+        dfree(draws);
         dfree(thermo_partial);
         dfree(thermo_out);
         dfree(d_gamma);
@@ -875,16 +878,9 @@ struct hm_system
         return method == 2 ? 3.0 * N : 3.0 * N - 3.0;
     }
 
-    void launch_step()
+    void fill_step_one(StepOneArgs& a1)
     {
-        // the Bussi factor needs the kinetic energy of every particle before step one: a
-        // step-begin kernel of its own. Without it, step one begins the step and step two ends it
         const bool bussi = method == 1;
-        if (bussi)
-            hchk(launch_step_begin(st, ke_partial, n_partial, 1, ndof(), dt, tau, kT, seed,
-                                   stream),
-                 "step begin");
-        StepOneArgs a1;
         memset(&a1, 0, sizeof(a1));
         a1.N = N;
         a1.pos = pos;
@@ -898,8 +894,7 @@ struct hm_system
         a1.pos32 = pos32;
         a1.use_state_alpha = bussi ? 1 : 0;
         a1.begin = bussi ? nullptr : st;
-        bool have_nl = rcut_max > 0.0;
-        if (have_nl)
+        if (rcut_max > 0.0)
         {
             a1.last = last;
             a1.maxsq = r_buff < 1e-6 ? -1.0 : distance_check_maxsq(rcut_max, r_buff);
@@ -910,17 +905,104 @@ struct hm_system
         }
         // the gather pair kernels read no cell list between builds: step one clears the
         // occupancy counters every step, which saves a launch; the cell-tiled kernels keep them
-        const int kind = pair_kind();
-        const bool fused_clear = have_nl && (kind == 1 || kind == 2);
-        if (fused_clear)
+        if (fused_clear())
         {
             a1.cell_size = cell_size;
             a1.ncell = ncell;
         }
-        hchk(launch_step_one(a1, stream), "step one");
-        if (have_nl)
+    }
+    bool fused_clear() const
+    {
+        return rcut_max > 0.0 && (pair_kind() == 1 || pair_kind() == 2);
+    }
+
+    void fill_step_two(StepTwoArgs& a2)
+    {
+        memset(&a2, 0, sizeof(a2));
+        a2.N = N;
+        a2.vel = vel;
+        a2.accel = accel;
+        a2.nforces = force_ptrs(a2.f);
+        a2.dt = dt;
+        a2.alpha = 1.0;
+        if (method == 2)
         {
-            if (!fused_clear)
+            a2.gamma_by_type = d_gamma;
+            a2.pos = pos;
+            a2.tag = tag;
+            a2.kT = kT;
+            a2.seed = seed;
+        }
+        a2.st = st;
+        a2.ke_partial = ke_partial;
+        a2.finish = st;
+    }
+
+    // room for the Bussi draws of a chunk of K steps (graphs hold its address)
+    void reserve_draws(unsigned int K)
+    {
+        if (method != 1 || K <= n_draws)
+            return;
+        hchk(hipStreamSynchronize(stream), "sync");
+        clear_graphs();
+        dfree(draws);
+        n_draws = 0;
+        draws = dalloc<BussiDraws>(std::max(K, 128u));
+        n_draws = std::max(K, 128u);
+    }
+
+    // K timesteps. Between two of them one launch takes the second half of the one and the first half
+    // of the other; the state that is copied, sorted or read exists only after the last.
+    void launch_steps(unsigned int K)
+    {
+        // the Bussi factor needs the kinetic energy of every particle before step one
+        const bool bussi = method == 1;
+        StepMidArgs m;
+        memset(&m, 0, sizeof(m));
+        fill_step_one(m.one);
+        fill_step_two(m.two);
+        m.st = st;
+        m.npartial = (N + 255) / 256;
+        m.ndof = ndof();
+        m.tau = tau;
+        m.kT = kT;
+        m.mode = !bussi ? MID_PLAIN
+                        : (m.npartial <= MID_SUM_MAX_PARTIAL ? MID_SUM : MID_ALPHA);
+        for (unsigned int k = 0; k < K; k++)
+        {
+            if (k == 0)
+            {
+                if (bussi)
+                {
+                    hchk(launch_bussi_draws(st, K, ndof(), seed, draws, stream), "Bussi draws");
+                    hchk(launch_step_begin(st, ke_partial, n_partial, 1, ndof(), dt, tau, kT, draws,
+                                           stream),
+                         "step begin");
+                }
+                hchk(launch_step_one(m.one, stream), "step one");
+            }
+            else
+            {
+                m.parity = (k - 1) & 1u;
+                m.draws = draws + k;
+                if (bussi)
+                    hchk(launch_ke(m, stream), "kinetic energy");
+                if (m.mode == MID_ALPHA)
+                    hchk(launch_step_begin(st, ke_partial, m.npartial, 1, ndof(), dt, tau, kT, m.draws,
+                                           stream),
+                         "step begin");
+                hchk(launch_step_mid(m, stream), "step");
+            }
+            launch_lists_and_forces();
+        }
+        hchk(launch_step_two(m.two, stream, nullptr), "step two");
+    }
+
+    void launch_lists_and_forces()
+    {
+        if (rcut_max > 0.0)
+        {
+            if (!fused_clear())
                 hchk(launch_cell_clear(ncell, cell_size, st, stream), "cell clear");
             if (N <= CELL_FUSED_MAX_N)
                 hchk(launch_cell_bin_rank(N, dim, cmax, pos, cell_size, last, &cond->cell_need,
@@ -940,35 +1022,13 @@ struct hm_system
             fill_nlist_args(k, true);
             hchk(launch_nlist_build(k, stream), "nlist build");
         }
+        struct InStep
         {
-            struct InStep
-            {
-                bool& f;
-                explicit InStep(bool& x) : f(x) { f = true; }
-                ~InStep() { f = false; }
-            } guard(in_step);
-            launch_forces(compute_virial);
-        }
-        StepTwoArgs a2;
-        memset(&a2, 0, sizeof(a2));
-        a2.N = N;
-        a2.vel = vel;
-        a2.accel = accel;
-        a2.nforces = force_ptrs(a2.f);
-        a2.dt = dt;
-        a2.alpha = 1.0;
-        if (method == 2)
-        {
-            a2.gamma_by_type = d_gamma;
-            a2.pos = pos;
-            a2.tag = tag;
-            a2.kT = kT;
-            a2.seed = seed;
-        }
-        a2.st = st;
-        a2.ke_partial = ke_partial;
-        a2.finish = bussi ? nullptr : st;
-        hchk(launch_step_two(a2, stream, nullptr), "step two");
+            bool& f;
+            explicit InStep(bool& x) : f(x) { f = true; }
+            ~InStep() { f = false; }
+        } guard(in_step);
+        launch_forces(compute_virial);
     }
 
     // ------------------------------------------------------------------ prep / forces
@@ -1351,10 +1411,10 @@ struct hm_system
     // ------------------------------------------------------------------ run
     void launch_chunk(unsigned int K)
     {
+        reserve_draws(K);
         if (!use_graph)
         {
-            for (unsigned int k = 0; k < K; k++)
-                launch_step();
+            launch_steps(K);
             return;
         }
         auto it = graphs.find(K);
@@ -1370,8 +1430,7 @@ struct hm_system
         hchk(hipStreamBeginCapture(stream, hipStreamCaptureModeThreadLocal), "begin capture");
         try
         {
-            for (unsigned int k = 0; k < K; k++)
-                launch_step();
+            launch_steps(K);
         }
         catch (...)
         {
@@ -1408,6 +1467,7 @@ struct hm_system
             const uint64_t ran = steps_run + (t - timestep);
             if (autotune && !retuned && !tune_cached && ran < retune_after)
                 K = std::min<uint64_t>(K, retune_after - ran);
+            reserve_draws((unsigned int)K);
             if (graphs.find((unsigned int)K) == graphs.end())
             {
                 graphs.emplace((unsigned int)K, capture_steps((unsigned int)K));

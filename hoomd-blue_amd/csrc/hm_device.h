@@ -202,25 +202,45 @@ HM_HD double gamma_dist(Philox& g, double m_alpha, double m_b)
     return v;
 }
 
-// BussiThermostat::compute_rescale_factor (hoomd/md/Thermostat.h:416-446).
-HM_HD double bussi_alpha(double K, double ndof, double dt, double tau, double kT,
-                         uint64_t timestep, uint16_t seed, uint32_t instance)
+// BussiThermostat::compute_rescale_factor (hoomd/md/Thermostat.h:416-446), in two parts: the random
+// draws of a step, which need no kinetic energy, and the factor from them.
+struct BussiDraws
+{
+    double r1, rg;
+};
+
+HM_HD BussiDraws bussi_draws(double ndof, uint64_t timestep, uint16_t seed, uint32_t instance)
+{
+#pragma clang fp contract(off)
+    Philox g(45, timestep, seed, instance);
+    BussiDraws d;
+    d.r1 = normal(g, 1.0, 0.0);
+    d.rg = 0.0;
+    if (ndof > 1.0)
+        d.rg = 2.0 * gamma_dist(g, (ndof - 1.0) / 2.0, 1.0);
+    return d;
+}
+
+HM_HD double bussi_factor(const BussiDraws& d, double K, double ndof, double dt, double tau, double kT)
 {
 #pragma clang fp contract(off)
     if (dt == 0.0 || ndof == 0)
         return 1.0;
-    Philox g(45, timestep, seed, instance);
     double c = 0.0;
     if (tau != 0.0)
         c = exp(-dt / tau);
-    double r1 = normal(g, 1.0, 0.0);
-    double rg = 0.0;
-    if (ndof > 1.0)
-        rg = 2.0 * gamma_dist(g, (ndof - 1.0) / 2.0, 1.0);
     double v = kT / 2.0 / K;
-    double term1 = v * (1.0 - c) * (rg + r1 * r1);
-    double term2 = 2.0 * r1 * sqrt(v * (1.0 - c) * c);
+    double term1 = v * (1.0 - c) * (d.rg + d.r1 * d.r1);
+    double term2 = 2.0 * d.r1 * sqrt(v * (1.0 - c) * c);
     return sqrt(c + term1 + term2);
+}
+
+HM_HD double bussi_alpha(double K, double ndof, double dt, double tau, double kT,
+                         uint64_t timestep, uint16_t seed, uint32_t instance)
+{
+    if (dt == 0.0 || ndof == 0)
+        return 1.0;
+    return bussi_factor(bussi_draws(ndof, timestep, seed, instance), K, ndof, dt, tau, kT);
 }
 
 // ------------------------------------------------------------------------------------ wave64

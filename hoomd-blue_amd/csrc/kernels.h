@@ -31,6 +31,9 @@ struct StepState
     unsigned long long forced_at;   // step of a forced build (sort, overflow recovery)
     unsigned long long shortest;    // shortest period between distance-check builds this run
     unsigned long long n_dangerous; // builds on the first check after a build with delay > 1
+    // current step as the step-mid kernels read it: kernel k of a chunk reads tick[k & 1], which it
+    // does not write, and leaves the step it begins in the other
+    unsigned long long tick[2];
 };
 
 enum : unsigned int
@@ -456,10 +459,42 @@ struct StepTwoArgs
 };
 hipError_t launch_step_two(const StepTwoArgs& a, hipStream_t s, unsigned int* nblocks_out);
 
-// step-begin kernel: advances the device timestep; Bussi factor from KE partial sums
+// Step two of a step and step one of the next in one launch, inside a chunk of steps: the velocity is
+// read and written once and the acceleration not at all (100 of 324 bytes per particle). The state
+// in between is never stored, so the first and the last step of a chunk keep the separate kernels.
+enum : int
+{
+    MID_PLAIN = 0,   // no thermostat factor (NVE, Langevin)
+    MID_ALPHA = 1,   // Bussi factor in StepState::alpha (ke_kernel, then step_begin_kernel)
+    MID_SUM = 2,     // every workgroup adds ke_kernel's partials and forms the factor
+};
+struct StepMidArgs
+{
+    StepOneArgs one;
+    StepTwoArgs two;
+    int mode;
+    unsigned int parity;     // of StepState::tick
+    StepState* st;
+    unsigned int npartial;
+    double ndof, tau, kT;    // Bussi
+    const BussiDraws* draws; // of the step that begins
+};
+// Adding up to 1 024 partials (8 KB) in every workgroup costs less than the launch it saves (the step at
+// 131 072 particles fell from 37.7 to 33.8 us with it and the fused launch); 4 096 would be 134 MB.
+constexpr unsigned int MID_SUM_MAX_PARTIAL = 1024;
+hipError_t launch_step_mid(const StepMidArgs& a, hipStream_t s);
+// Kinetic-energy partials of the velocities after step two (which are not stored)
+hipError_t launch_ke(const StepMidArgs& a, hipStream_t s);
+// Bussi draws of the next n steps: one thread each, so that a chunk waits once for their long FP64 chain
+// (about 6 us) and not every step
+hipError_t launch_bussi_draws(const StepState* st, unsigned int n, double ndof, uint16_t seed,
+                              BussiDraws* draws, hipStream_t s);
+
+// step-begin kernel: advances the device timestep; Bussi factor from KE partial sums and the
+// step's draws
 hipError_t launch_step_begin(StepState* st, const double* ke_partial, unsigned int npartial,
                              int bussi, double ndof, double dt, double tau, double kT,
-                             uint16_t seed, hipStream_t s);
+                             const BussiDraws* draws, hipStream_t s);
 hipError_t launch_set_rebuild(StepState* st, hipStream_t s);  // rebuild before next forces
 
 // initial accelerations a = F/m (IntegratorTwoStep::prepRun -> computeAccelerations)

@@ -2562,78 +2562,96 @@ hipError_t launch_bond_index(unsigned int N, const unsigned int* tag, const unsi
 // TwoStepConstantVolume::integrateStepOne (hoomd/md/TwoStepConstantVolume.cc:7-80), fused with
 // NeighborList::distanceCheck for step t + 1 (NeighborList.cc:1220-1289) and with clearing the
 // cell occupancy counters for a possible rebuild.
+//
+// Drift of particle n with its rescaled velocity: new position, image (read and written only when the
+// particle crosses the box), relative and FP32 copies; returns whether it moved past the buffer.
+__device__ __forceinline__ bool drift_particle(const StepOneArgs& a, unsigned int n, double4 p,
+                                               double vx, double vy, double vz)
+{
+#pragma clang fp contract(off)
+    const double dt = a.dt;
+    double px = p.x + dt * vx;
+    double py = p.y + dt * vy;
+    double pz = p.z + dt * vz;
+    i3 d{0, 0, 0};
+    wrap_axis(px, d.x, a.box.lo[0], a.box.hi[0], a.box.L[0]);
+    wrap_axis(py, d.y, a.box.lo[1], a.box.hi[1], a.box.L[1]);
+    wrap_axis(pz, d.z, a.box.lo[2], a.box.hi[2], a.box.L[2]);
+    p.x = px;
+    p.y = py;
+    p.z = pz;
+    a.pos[n] = p;
+    if (d.x || d.y || d.z)
+    {
+        i3 img = a.image[n];
+        img.x += d.x;
+        img.y += d.y;
+        img.z += d.z;
+        a.image[n] = img;
+    }
+    if (a.pos32)
+        a.pos32[n] = make_float4((float)px, (float)py, (float)pz, 0.f);
+    if (a.rel.rel)
+    {
+        const float4 r = rel_of(px, py, pz, a.rel.pcell[n], a.box, a.rel);
+        a.rel.rel[a.rel.slot_of[n]] = make_float3(r.x, r.y, r.z);
+    }
+    if (!a.last)
+        return false;
+    const d3 l = a.last[n];
+    double dx = px - 1.0 * l.x, dy = py - 1.0 * l.y, dz = pz - 1.0 * l.z;
+    min_image(a.box, dx, dy, dz);
+    return dx * dx + dy * dy + dz * dz >= a.maxsq;
+}
+
+// NeighborList::needsUpdating (NeighborList.cc:1325-1418) for step t1: no check before
+// rebuild_check_delay steps have passed since the last build; an unconditional build when the
+// buffer is zero or distance checks are off and the period is hit; else the distance check. The
+// conditions are the same on every lane, so the ballot stays uniform.
+__device__ __forceinline__ void flag_rebuild(const StepOneArgs& a, unsigned long long t1, bool moved)
+{
+    const StepState* st = a.flag_state;
+    const bool should = !(t1 < st->last_update + a.check_delay);
+    const bool always = a.maxsq < 0.0
+                        || (!a.dist_check
+                            && (a.check_delay == 0
+                                || (a.check_delay > 1 && t1 == st->last_update + a.check_delay)));
+    if (should && (always || __ballot(moved) != 0) && (threadIdx.x & 63u) == 0)
+        atomicMax(&a.flag_state->rebuild_at, t1);
+}
+
+__device__ __forceinline__ void clear_cells(const StepOneArgs& a, unsigned int gtid, unsigned int nthreads)
+{
+    if (a.cell_size)
+        for (unsigned int c = gtid; c < a.ncell; c += nthreads)
+            a.cell_size[c] = 0;
+}
+
 __global__ __launch_bounds__(256) void step_one_kernel(StepOneArgs a)
 {
 #pragma clang fp contract(off)
-    const unsigned int gtid = blockIdx.x * blockDim.x + threadIdx.x;
-    if (a.cell_size)
-        for (unsigned int c = gtid; c < a.ncell; c += gridDim.x * blockDim.x)
-            a.cell_size[c] = 0;
-    const unsigned int n = gtid;
+    const unsigned int n = blockIdx.x * blockDim.x + threadIdx.x;
+    clear_cells(a, n, gridDim.x * blockDim.x);
     bool moved = false;
     if (n < a.N)
     {
         const double alpha = (a.st && a.use_state_alpha) ? a.st->alpha : a.alpha;
         const double dt = a.dt;
         double4 v = a.vel[n];
-        double4 p = a.pos[n];
         const d3 acc = a.accel[n];
-        i3 img = a.image[n];
-        double vx = v.x + (1.0 / 2.0) * acc.x * dt;
-        double vy = v.y + (1.0 / 2.0) * acc.y * dt;
-        double vz = v.z + (1.0 / 2.0) * acc.z * dt;
-        vx *= alpha;
-        vy *= alpha;
-        vz *= alpha;
-        double px = p.x + dt * vx;
-        double py = p.y + dt * vy;
-        double pz = p.z + dt * vz;
-        wrap_axis(px, img.x, a.box.lo[0], a.box.hi[0], a.box.L[0]);
-        wrap_axis(py, img.y, a.box.lo[1], a.box.hi[1], a.box.L[1]);
-        wrap_axis(pz, img.z, a.box.lo[2], a.box.hi[2], a.box.L[2]);
-        v.x = vx;
-        v.y = vy;
-        v.z = vz;
-        p.x = px;
-        p.y = py;
-        p.z = pz;
+        v.x = (v.x + (1.0 / 2.0) * acc.x * dt) * alpha;
+        v.y = (v.y + (1.0 / 2.0) * acc.y * dt) * alpha;
+        v.z = (v.z + (1.0 / 2.0) * acc.z * dt) * alpha;
         a.vel[n] = v;
-        a.pos[n] = p;
-        a.image[n] = img;
-        if (a.pos32)
-            a.pos32[n] = make_float4((float)px, (float)py, (float)pz, 0.f);
-        if (a.rel.rel)
-        {
-            const float4 r = rel_of(px, py, pz, a.rel.pcell[n], a.box, a.rel);
-            a.rel.rel[a.rel.slot_of[n]] = make_float3(r.x, r.y, r.z);
-        }
-        if (a.last)
-        {
-            const d3 l = a.last[n];
-            double dx = px - 1.0 * l.x, dy = py - 1.0 * l.y, dz = pz - 1.0 * l.z;
-            min_image(a.box, dx, dy, dz);
-            moved = dx * dx + dy * dy + dz * dz >= a.maxsq;
-        }
+        moved = drift_particle(a, n, a.pos[n], v.x, v.y, v.z);
     }
-    if (a.begin && gtid == 0)
-        a.begin->timestep = a.begin->next;
-    if (a.flag_state)
+    if (a.begin && n == 0)
     {
-        // NeighborList::needsUpdating (NeighborList.cc:1325-1418) for step t1: no check before
-        // rebuild_check_delay steps have passed since the last build; an unconditional build when
-        // the buffer is zero or distance checks are off and the period is hit; else the distance
-        // check. The conditions are the same on every lane, so the ballot stays uniform.
-        const StepState* st = a.flag_state;
-        const unsigned long long t1 = (a.begin ? a.begin->next : st->timestep) + 1;
-        const bool should = !(t1 < st->last_update + a.check_delay);
-        const bool always = a.maxsq < 0.0
-                            || (!a.dist_check
-                                && (a.check_delay == 0
-                                    || (a.check_delay > 1
-                                        && t1 == st->last_update + a.check_delay)));
-        if (should && (always || __ballot(moved) != 0) && (threadIdx.x & 63u) == 0)
-            atomicMax(&a.flag_state->rebuild_at, t1);
+        a.begin->timestep = a.begin->next;
+        a.begin->tick[0] = a.begin->next;
     }
+    if (a.flag_state)
+        flag_rebuild(a, (a.begin ? a.begin->next : a.flag_state->timestep) + 1, moved);
 }
 
 hipError_t launch_step_one(const StepOneArgs& a, hipStream_t s)
@@ -2668,6 +2686,57 @@ __device__ __forceinline__ double block_sum_256(double v, double* sh)
 // TwoStepConstantVolume::integrateStepTwo (TwoStepConstantVolume.cc:213-260) or
 // TwoStepLangevin::integrateStepTwo (hoomd/md/TwoStepLangevin.cc:206-275), with the net force
 // summed from up to four force arrays and the FP64 kinetic-energy partial of each block.
+__device__ __forceinline__ float4 first_force(const StepTwoArgs& a, unsigned int n)
+{
+    return a.nforces ? a.f[0][n] : make_float4(0.f, 0.f, 0.f, 0.f);
+}
+
+// Second half kick of particle n at step t: v becomes the full-step velocity, the acceleration is
+// returned. f0: its first force
+template<bool LANGEVIN>
+__device__ __forceinline__ d3 second_kick(const StepTwoArgs& a, unsigned int n, uint64_t t, double4& v,
+                                          float4 f0)
+{
+#pragma clang fp contract(off)
+    const double minv = 1.0 / v.w;
+    double Fx = (double)f0.x, Fy = (double)f0.y, Fz = (double)f0.z;
+    for (unsigned int q = 1; q < a.nforces; q++)
+    {
+        const float4 f = a.f[q][n];
+        Fx += (double)f.x;
+        Fy += (double)f.y;
+        Fz += (double)f.z;
+    }
+    d3 ac;
+    if (LANGEVIN)
+    {
+        Philox g(25, t, a.seed, a.tag[n]);
+        const double rx = uniform(g, -1.0, 1.0);
+        const double ry = uniform(g, -1.0, 1.0);
+        const double rz = uniform(g, -1.0, 1.0);
+        const double gm = a.gamma_by_type[(unsigned int)a.pos[n].w];
+        const double coeff = sqrt(6.0 * gm * a.kT / a.dt);
+        const double bx = rx * coeff - gm * v.x;
+        const double by = ry * coeff - gm * v.y;
+        const double bz = rz * coeff - gm * v.z;
+        ac = d3{(Fx + bx) * minv, (Fy + by) * minv, (Fz + bz) * minv};
+        v.x += (1.0 / 2.0) * ac.x * a.dt;
+        v.y += (1.0 / 2.0) * ac.y * a.dt;
+        v.z += (1.0 / 2.0) * ac.z * a.dt;
+    }
+    else
+    {
+        ac = d3{Fx * minv, Fy * minv, Fz * minv};
+        v.x *= a.alpha;
+        v.y *= a.alpha;
+        v.z *= a.alpha;
+        v.x += (1.0 / 2.0) * a.dt * ac.x;
+        v.y += (1.0 / 2.0) * a.dt * ac.y;
+        v.z += (1.0 / 2.0) * a.dt * ac.z;
+    }
+    return ac;
+}
+
 template<bool LANGEVIN>
 __global__ __launch_bounds__(256) void step_two_kernel(StepTwoArgs a)
 {
@@ -2678,51 +2747,11 @@ __global__ __launch_bounds__(256) void step_two_kernel(StepTwoArgs a)
     if (n < a.N)
     {
         double4 v = a.vel[n];
-        const double m = v.w;
-        const double minv = 1.0 / m;
-        double Fx = 0.0, Fy = 0.0, Fz = 0.0;
-        for (unsigned int q = 0; q < a.nforces; q++)
-        {
-            const float4 f = a.f[q][n];
-            Fx += (double)f.x;
-            Fy += (double)f.y;
-            Fz += (double)f.z;
-        }
-        double ax, ay, az;
-        if (LANGEVIN)
-        {
-            const uint64_t t = a.st ? a.st->timestep : a.timestep;
-            Philox g(25, t, a.seed, a.tag[n]);
-            const double rx = uniform(g, -1.0, 1.0);
-            const double ry = uniform(g, -1.0, 1.0);
-            const double rz = uniform(g, -1.0, 1.0);
-            const double gm = a.gamma_by_type[(unsigned int)a.pos[n].w];
-            const double coeff = sqrt(6.0 * gm * a.kT / a.dt);
-            const double bx = rx * coeff - gm * v.x;
-            const double by = ry * coeff - gm * v.y;
-            const double bz = rz * coeff - gm * v.z;
-            ax = (Fx + bx) * minv;
-            ay = (Fy + by) * minv;
-            az = (Fz + bz) * minv;
-            v.x += (1.0 / 2.0) * ax * a.dt;
-            v.y += (1.0 / 2.0) * ay * a.dt;
-            v.z += (1.0 / 2.0) * az * a.dt;
-        }
-        else
-        {
-            ax = Fx * minv;
-            ay = Fy * minv;
-            az = Fz * minv;
-            v.x *= a.alpha;
-            v.y *= a.alpha;
-            v.z *= a.alpha;
-            v.x += (1.0 / 2.0) * a.dt * ax;
-            v.y += (1.0 / 2.0) * a.dt * ay;
-            v.z += (1.0 / 2.0) * a.dt * az;
-        }
+        const d3 ac = second_kick<LANGEVIN>(a, n, a.st ? a.st->timestep : a.timestep, v,
+                                             first_force(a, n));
         a.vel[n] = v;
-        a.accel[n] = d3{ax, ay, az};
-        ke = m * (v.x * v.x + v.y * v.y + v.z * v.z);
+        a.accel[n] = ac;
+        ke = v.w * (v.x * v.x + v.y * v.y + v.z * v.z);
     }
     if (a.ke_partial)
     {
@@ -2732,6 +2761,128 @@ __global__ __launch_bounds__(256) void step_two_kernel(StepTwoArgs a)
     }
     if (a.finish && n == 0)
         a.finish->next = a.finish->timestep + 1;
+}
+
+// Kinetic energy after step two, per 256 particles
+__global__ __launch_bounds__(256) void ke_kernel(StepMidArgs m)
+{
+#pragma clang fp contract(off)
+    __shared__ double sh[4];
+    const unsigned int n = blockIdx.x * 256u + threadIdx.x;
+    double ke = 0.0;
+    if (n < m.two.N)
+    {
+        double4 v = m.two.vel[n];
+        second_kick<false>(m.two, n, 0, v, first_force(m.two, n));
+        ke = v.w * (v.x * v.x + v.y * v.y + v.z * v.z);
+    }
+    const double t = block_sum_256(ke, sh);
+    if (threadIdx.x == 0)
+        m.two.ke_partial[blockIdx.x] = t;
+}
+
+hipError_t launch_ke(const StepMidArgs& a, hipStream_t s)
+{
+    if (a.npartial == 0)
+        return hipSuccess;
+    hipLaunchKernelGGL(ke_kernel, dim3(a.npartial), dim3(256), 0, s, a);
+    return hipGetLastError();
+}
+
+__global__ __launch_bounds__(64) void bussi_draws_kernel(const StepState* st, unsigned int n,
+                                                         double ndof, uint16_t seed,
+                                                         BussiDraws* draws)
+{
+    const unsigned int k = blockIdx.x * 64u + threadIdx.x;
+    if (k < n)
+        draws[k] = bussi_draws(ndof, st->next + k, seed, 0u);
+}
+
+hipError_t launch_bussi_draws(const StepState* st, unsigned int n, double ndof, uint16_t seed,
+                              BussiDraws* draws, hipStream_t s)
+{
+    if (n == 0)
+        return hipSuccess;
+    hipLaunchKernelGGL(bussi_draws_kernel, dim3((n + 63) / 64), dim3(64), 0, s, st, n, ndof, seed, draws);
+    return hipGetLastError();
+}
+
+// Step two of step t and step one of t + 1 (StepMidArgs). HBM-bound: at 1 048 576 particles 38 us (and
+// 11 for the kinetic energy of the Bussi factor) where the two kernels took 42 + 23, about 5 TB/s; for
+// 10^6 beads under Langevin 51 us, before 47 + 30. At a few thousand particles it is a launch fewer.
+template<bool LANGEVIN, int MODE>
+__global__ __launch_bounds__(256) void step_mid_kernel(StepMidArgs m)
+{
+#pragma clang fp contract(off)
+    __shared__ double sh[4];
+    __shared__ double factor;
+    const unsigned int n = blockIdx.x * 256u + threadIdx.x;
+    const unsigned long long t = MODE == MID_ALPHA ? 0ull : m.st->tick[m.parity];
+    double alpha = 1.0;
+    if (MODE == MID_ALPHA)
+        alpha = m.st->alpha;
+    if (MODE == MID_SUM)
+    {
+        // the order of step_begin_kernel
+        double acc = 0.0;
+        for (unsigned int q = threadIdx.x; q < m.npartial; q += 256)
+            acc += m.two.ke_partial[q];
+        const double tot = block_sum_256(acc, sh);
+        if (threadIdx.x == 0)
+        {
+            const double K = tot * 0.5;
+            double f = 1.0;
+            if (K == 0.0)
+            {
+                if (blockIdx.x == 0)
+                    atomicOr(&m.st->error, (unsigned int)ERR_ZERO_KE);
+            }
+            else
+                f = bussi_factor(*m.draws, K, m.ndof, m.one.dt, m.tau, m.kT);
+            factor = f;
+        }
+        __syncthreads();
+        alpha = factor;
+    }
+    clear_cells(m.one, n, gridDim.x * 256u);
+    bool moved = false;
+    if (n < m.one.N)
+    {
+        double4 v = m.one.vel[n];
+        const double dt = m.one.dt;
+        const d3 acc = second_kick<LANGEVIN>(m.two, n, t, v, first_force(m.two, n));
+        v.x = (v.x + (1.0 / 2.0) * acc.x * dt) * alpha;
+        v.y = (v.y + (1.0 / 2.0) * acc.y * dt) * alpha;
+        v.z = (v.z + (1.0 / 2.0) * acc.z * dt) * alpha;
+        m.one.vel[n] = v;
+        moved = drift_particle(m.one, n, m.one.pos[n], v.x, v.y, v.z);
+    }
+    if (MODE != MID_ALPHA && n == 0)
+    {
+        m.st->timestep = t + 1;
+        m.st->tick[m.parity ^ 1u] = t + 1;
+        m.st->alpha = alpha;
+    }
+    if (m.one.flag_state)
+        flag_rebuild(m.one, MODE == MID_ALPHA ? m.st->timestep + 1 : t + 2, moved);
+}
+
+hipError_t launch_step_mid(const StepMidArgs& a, hipStream_t s)
+{
+    if (a.one.N == 0)
+        return hipSuccess;
+    const unsigned int blocks = (a.one.N + 255) / 256;
+    if (a.npartial != blocks || a.one.N != a.two.N || !a.st)
+        return hipErrorInvalidValue;
+    if (a.two.gamma_by_type)
+        hipLaunchKernelGGL((step_mid_kernel<true, MID_PLAIN>), dim3(blocks), dim3(256), 0, s, a);
+    else if (a.mode == MID_PLAIN)
+        hipLaunchKernelGGL((step_mid_kernel<false, MID_PLAIN>), dim3(blocks), dim3(256), 0, s, a);
+    else if (a.mode == MID_ALPHA)
+        hipLaunchKernelGGL((step_mid_kernel<false, MID_ALPHA>), dim3(blocks), dim3(256), 0, s, a);
+    else
+        hipLaunchKernelGGL((step_mid_kernel<false, MID_SUM>), dim3(blocks), dim3(256), 0, s, a);
+    return hipGetLastError();
 }
 
 hipError_t launch_step_two(const StepTwoArgs& a, hipStream_t s, unsigned int* nblocks_out)
@@ -2781,7 +2932,7 @@ hipError_t launch_ke_partial(unsigned int N, const double4* vel, double* partial
 __global__ __launch_bounds__(256) void step_begin_kernel(StepState* st, const double* ke_partial,
                                                          unsigned int npartial, int bussi,
                                                          double ndof, double dt, double tau,
-                                                         double kT, uint16_t seed)
+                                                         double kT, const BussiDraws* draws)
 {
 #pragma clang fp contract(off)
     __shared__ double sh[4];
@@ -2795,6 +2946,7 @@ __global__ __launch_bounds__(256) void step_begin_kernel(StepState* st, const do
         const unsigned long long t = st->next;
         st->timestep = t;
         st->next = t + 1;
+        st->tick[0] = t;
         double alpha = 1.0;
         if (bussi)
         {
@@ -2802,7 +2954,7 @@ __global__ __launch_bounds__(256) void step_begin_kernel(StepState* st, const do
             if (K == 0.0)
                 st->error |= ERR_ZERO_KE;
             else
-                alpha = bussi_alpha(K, ndof, dt, tau, kT, t, seed, 0u);
+                alpha = bussi_factor(*draws, K, ndof, dt, tau, kT);
         }
         st->alpha = alpha;
     }
@@ -2810,10 +2962,10 @@ __global__ __launch_bounds__(256) void step_begin_kernel(StepState* st, const do
 
 hipError_t launch_step_begin(StepState* st, const double* ke_partial, unsigned int npartial,
                              int bussi, double ndof, double dt, double tau, double kT,
-                             uint16_t seed, hipStream_t s)
+                             const BussiDraws* draws, hipStream_t s)
 {
     hipLaunchKernelGGL(step_begin_kernel, dim3(1), dim3(256), 0, s, st, ke_partial, npartial,
-                       bussi, ndof, dt, tau, kT, seed);
+                       bussi, ndof, dt, tau, kT, draws);
     return hipGetLastError();
 }
 
