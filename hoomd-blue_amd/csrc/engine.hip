@@ -16,6 +16,7 @@
 #include <cmath>
 #include <cstdio>
 #include <cstring>
+#include <functional>
 #include <map>
 #include <new>
 #include <stdexcept>
@@ -224,6 +225,9 @@ struct hm_system
     // run control
     uint64_t timestep = 0;
     bool prepared = false;
+    // the lists, capacities and launch shapes of the present forces are set up: what a training frame
+    // needs, whose positions replace the state's (a run prepares again)
+    bool configured = false;
     int compute_virial = 0;
     // FP32 copy of the positions for the learned-CG pair passes (allocated with the first such
     // force); written by step one, so inside a step the forces read it as it is
@@ -1032,6 +1036,44 @@ struct hm_system
     }
 
     // ------------------------------------------------------------------ prep / forces
+    // the launches of a complete list build; conditions gather what they found
+    void launch_list_build()
+    {
+        hchk(launch_cell_clear(ncell, cell_size, nullptr, stream), "clear cells");
+        hchk(launch_cell_build(N, pos, box, dim, cmax, cell_size, nullptr, last, &cond->cell_need,
+                               nullptr, stream, ckey, chome),
+             "cell build");
+        hchk(launch_cell_rank(N, cmax, pos, cell_size, ckey, chome, entries, cell_idx, nullptr,
+                              stream, box, rel_frame()),
+             "cell order");
+        NlistKernelArgs k;
+        fill_nlist_args(k, false);
+        k.counter = nullptr;
+        hchk(launch_nlist_build(k, stream), "nlist build");
+    }
+
+    // What the list builds since the last clear found, read on the host: true when every list fits;
+    // otherwise the capacities are grown and the builds have to be repeated. An overflowed build
+    // leaves short but valid rows, so work launched after it stays in bounds.
+    bool lists_fit()
+    {
+        hchk(hipMemcpyAsync(h_cond, cond, sizeof(Conditions), hipMemcpyDeviceToHost, stream),
+             "read conditions");
+        hchk(hipStreamSynchronize(stream), "sync");
+        const Conditions c = *h_cond;
+        if (c.nan_idx)
+            throw HmError{HM_ERR_NAN, "particle position is NaN"};
+        if (c.out_idx)
+            throw HmError{HM_ERR_OUTSIDE, "particle is no longer in the simulation box"};
+        if (c.cell_need > cmax)
+            grow_cmax(c.cell_need);
+        else if (c.nlist_need > nmax)
+            grow_nmax(c.nlist_need);
+        else
+            return true;
+        return false;
+    }
+
     void build_nlist_now()
     {
         // CellList::compute + NeighborList::compute loops with host-side regrow (the reference's
@@ -1039,38 +1081,9 @@ struct hm_system
         for (int attempt = 0; attempt < 64; attempt++)
         {
             hchk(hipMemsetAsync(cond, 0, sizeof(Conditions), stream), "clear conditions");
-            hchk(hipMemsetAsync(cell_size, 0, sizeof(unsigned int) * ncell, stream), "clear cells");
-            hchk(launch_cell_build(N, pos, box, dim, cmax, cell_size, nullptr, last,
-                                   &cond->cell_need, nullptr, stream, ckey, chome),
-                 "cell build");
-            hchk(hipMemcpyAsync(h_cond, cond, sizeof(Conditions), hipMemcpyDeviceToHost, stream),
-                 "read conditions");
-            hchk(hipStreamSynchronize(stream), "sync");
-            if (h_cond->nan_idx)
-                throw HmError{HM_ERR_NAN, "particle position is NaN"};
-            if (h_cond->out_idx)
-                throw HmError{HM_ERR_OUTSIDE, "particle is no longer in the simulation box"};
-            if (h_cond->cell_need > cmax)
-            {
-                grow_cmax(h_cond->cell_need);
-                continue;
-            }
-            hchk(launch_cell_rank(N, cmax, pos, cell_size, ckey, chome, entries, cell_idx, nullptr,
-                                  stream, box, rel_frame()),
-                 "cell order");
-            NlistKernelArgs k;
-            fill_nlist_args(k, false);
-            k.counter = nullptr;
-            hchk(launch_nlist_build(k, stream), "nlist build");
-            hchk(hipMemcpyAsync(h_cond, cond, sizeof(Conditions), hipMemcpyDeviceToHost, stream),
-                 "read conditions");
-            hchk(hipStreamSynchronize(stream), "sync");
-            if (h_cond->nlist_need > nmax)
-            {
-                grow_nmax(h_cond->nlist_need);
-                continue;
-            }
-            return;
+            launch_list_build();
+            if (lists_fit())
+                return;
         }
         throw HmError{HM_ERR_LAUNCH, "neighbour list did not converge"};
     }
@@ -1318,6 +1331,7 @@ struct hm_system
         hchk(hipStreamSynchronize(stream), "prep sync");
         check_errors_after(false);
         prepared = true;
+        configured = true;
     }
 
     void check_errors_after(bool chunk)
@@ -1679,6 +1693,7 @@ int hm_sys_set_nlist(hm_system* s, double r_buff, int exclude_bonds)
     s->r_buff = r_buff;
     s->exclude_bonds = exclude_bonds;
     s->prepared = false;
+    s->configured = false;
     s->nmax = 0;
     s->clear_graphs();
     return HM_OK;
@@ -1706,6 +1721,7 @@ int hm_sys_add_pair_lj(hm_system* s, const double* r_cut, const double* r_on,
         hchk(hipMemset(f.v, 0, sizeof(float) * 6 * s->N), "clear");
         s->forces.push_back(f);
         s->prepared = false;
+        s->configured = false;
         s->nmax = 0;
         s->clear_graphs();
         return (int)s->forces.size() - 1;
@@ -1757,6 +1773,7 @@ int hm_sys_add_pair_table(hm_system* s, const double* r_cut, const double* r_min
         hchk(hipMemset(f.v, 0, sizeof(float) * 6 * s->N), "clear");
         s->forces.push_back(f);
         s->prepared = false;
+        s->configured = false;
         s->nmax = 0;
         s->clear_graphs();
         return (int)s->forces.size() - 1;
@@ -1869,6 +1886,7 @@ int add_bond_force(hm_system* s, unsigned int nb, const unsigned int* bond_tags,
         }
         s->forces.push_back(f);
         s->prepared = false;
+        s->configured = false;
         s->clear_graphs();
         return (int)s->forces.size() - 1;
     });
@@ -1988,6 +2006,7 @@ int hm_sys_set_pair_kernel(hm_system* s, int kind, unsigned int tpp, unsigned in
     s->pair_kernel_kind = kind;
     // the relative positions of kind 2 are written by the cell-list build: build again
     s->prepared = false;
+    s->configured = false;
     // tpp = size = 0: the autotuner picks the launch configuration at the next run
     s->autotune = tpp == 0 && size == 0;
     s->pair_tuned = false;
@@ -2018,7 +2037,7 @@ int hm_sys_set_autotune(hm_system* s, int on)
     s->autotune = on != 0;
     s->pair_tuned = false;
     if (s->autotune)
-        s->prepared = false;
+        s->prepared = s->configured = false;
     return HM_OK;
 }
 
@@ -2440,16 +2459,23 @@ void mlp_build_now(hm_system* s)
         s->build_nlist_now();
 }
 
-// one training frame: positions and targets in, list built, forces, loss and gradient rows
+// Set up for training frames. A full prep also evaluates the forces, accelerations and energy of the
+// present state, which a frame replaces; it runs once for a configuration.
+void mlp_prepare_frames(hm_system* s)
+{
+    if (s->method < 0 || !s->configured)
+        s->prep();
+}
+
+// one training frame: positions and targets in, list built, forces, loss and gradient rows. Nothing is
+// read on the host: the caller checks lists_fit() before it uses the result.
 void mlp_frame_pass(hm_system* s, ForceSlot& f, const float* fpos, const float* fforce,
                     double* loss_out)
 {
-    if (!s->prepared)
-        s->prep();
     hchk(launch_mlp_load_frame(s->N, s->rtag, fpos, fforce, s->box, s->pos, f.mT, s->stream),
          "mlp load frame");
     if (s->rcut_max > 0.0)
-        s->build_nlist_now();
+        s->launch_list_build();
     MlpArgs a = s->mlp_args(f, 0);
     // training reads the FP32 dE/dG: the loss and its gradient are those of the FP32 forces
     // (the bf16 copy of the production force pass moves forces by about 1e-3 of their size,
@@ -2460,6 +2486,19 @@ void mlp_frame_pass(hm_system* s, ForceSlot& f, const float* fpos, const float* 
     hchk(launch_mlp_force(a, true, s->stream), "mlp forces");
     hchk(launch_mlp_backward(a, s->stream), "mlp backward");
     hchk(launch_mlp_loss(f.mLoss, mlp_pair_blocks(s->N), loss_out, s->stream), "mlp loss");
+}
+
+// frames: a function that launches frame passes; repeated until the lists of all of them fit
+void mlp_until_fit(hm_system* s, const std::function<void()>& frames)
+{
+    for (int attempt = 0; attempt < 64; attempt++)
+    {
+        hchk(hipMemsetAsync(s->cond, 0, sizeof(Conditions), s->stream), "clear conditions");
+        frames();
+        if (s->lists_fit())
+            return;
+    }
+    throw HmError{HM_ERR_LAUNCH, "neighbour list did not converge"};
 }
 } // namespace
 
@@ -2493,6 +2532,7 @@ int hm_sys_add_mlp_cg(hm_system* s, const hm_mlp_cg_model* model, const float* p
         hchk(hipStreamSynchronize(s->stream), "sync");
         s->forces.push_back(f);
         s->prepared = false;
+        s->configured = false;
         s->nmax = 0;
         s->clear_graphs();
         return (int)s->forces.size() - 1;
@@ -2654,16 +2694,18 @@ int hm_sys_mlp_loss_grad(hm_system* s, int force_id, const float* frame_pos,
         mlp_alloc_training(s, *f);
         if (!f->mLossOut)
             f->mLossOut = dalloc<double>(1);
-        mlp_frame_pass(s, *f, frame_pos, frame_force, f->mLossOut);
-        hchk(launch_mlp_grad_sum(f->mGpart, f->mGrad, s->stream), "mlp gradient");
-        hchk(hipStreamSynchronize(s->stream), "sync");
+        mlp_prepare_frames(s);
+        s->prepared = false;  // the next run starts from the frame's positions: prepare again
+        mlp_until_fit(s, [&]() {
+            mlp_frame_pass(s, *f, frame_pos, frame_force, f->mLossOut);
+            hchk(launch_mlp_grad_sum(f->mGpart, f->mGrad, s->stream), "mlp gradient");
+        });
         double sq = 0.0;
         hchk(hipMemcpy(&sq, f->mLossOut, sizeof(double), hipMemcpyDeviceToHost), "download");
         *loss = sq / (3.0 * (double)s->N);
         if (grad)
             hchk(hipMemcpy(grad, f->mGrad, sizeof(float) * MLP_NPARAM, hipMemcpyDeviceToHost),
                  "download");
-        s->prepared = false;
         return HM_OK;
     });
 }
@@ -2687,18 +2729,23 @@ int hm_sys_mlp_train(hm_system* s, int force_id, const hm_mlp_train_args* t)
         if (B > 1 && !f->mGacc)
             f->mGacc = dalloc<float>(MLP_NPARAM);
         const size_t stride = (size_t)3 * s->N;
+        mlp_prepare_frames(s);
+        s->prepared = false;  // the next run starts from the frame's positions: prepare again
         for (unsigned int k = 0; k < t->nsteps; k++)
         {
-            for (unsigned int b = 0; b < B; b++)
-            {
-                const size_t q = (size_t)k * B + b;
-                const unsigned int fr = t->order ? t->order[q] : (unsigned int)(q % t->nframes);
-                mlp_frame_pass(s, *f, t->frame_pos + stride * fr, t->frame_force + stride * fr,
-                               f->mLossOut + q);
-                if (B > 1)
-                    hchk(launch_mlp_grad_accum(f->mGpart, f->mGacc, b == 0, s->stream),
-                         "mlp gradient sum");
-            }
+            // one look at the conditions for all frames of the step, before its update
+            mlp_until_fit(s, [&]() {
+                for (unsigned int b = 0; b < B; b++)
+                {
+                    const size_t q = (size_t)k * B + b;
+                    const unsigned int fr = t->order ? t->order[q] : (unsigned int)(q % t->nframes);
+                    mlp_frame_pass(s, *f, t->frame_pos + stride * fr, t->frame_force + stride * fr,
+                                   f->mLossOut + q);
+                    if (B > 1)
+                        hchk(launch_mlp_grad_accum(f->mGpart, f->mGacc, b == 0, s->stream),
+                             "mlp gradient sum");
+                }
+            });
             if (B > 1)
                 hchk(launch_mlp_adam_acc(f->mparams, f->mM1, f->mM2, f->mGacc, 1.0f / (float)B,
                                          f->mbf16, (float)t->lr, (float)t->beta1,
@@ -2725,7 +2772,6 @@ int hm_sys_mlp_train(hm_system* s, int force_id, const hm_mlp_train_args* t)
                 t->loss[k] = sum / B / (3.0 * (double)s->N);
             }
         }
-        s->prepared = false;
         return HM_OK;
     });
 }
