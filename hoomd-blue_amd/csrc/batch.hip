@@ -37,6 +37,7 @@
 
 #include "capi_util.h"
 #include "evaluators.h"
+#include "kernel_util.h"
 #include "kernels.h"
 
 using namespace hm;
@@ -310,7 +311,9 @@ __global__ __launch_bounds__(BTILE) void bcell_bin_kernel(
     cellc[p] = cc;
     if (R.dim >= REL_MIN_DIM)
         rel[p] = centre_rel(x, cc, R);
-    const unsigned int slot = atomicAdd(&cell_size[c], 1u);
+    // consecutive particles mostly share a cell: one atomic for a run of lanes (1.3e6 particles of 256
+    // replicas, a tenth of them rebuilding: 9.9 us, one atomic a particle 36)
+    const unsigned int slot = claim_slot(c, true, cell_size);
     if (slot < cmax)
         cell_raw[(size_t)c * cmax + slot] = p;
     else
@@ -391,7 +394,7 @@ __global__ __launch_bounds__(64 * NL_WAVES) void bnlist_kernel(
     const Rep* __restrict__ reps, const unsigned int* __restrict__ cell_rep,
     const RepState* __restrict__ rst, const double4* __restrict__ pos, unsigned int cmax,
     const unsigned int* __restrict__ cell_size, const unsigned int* __restrict__ cell_idx,
-    double rlistsq, unsigned int nmax, unsigned int* __restrict__ nlist,
+    double rlistsq, unsigned int nmax, unsigned int stride, unsigned int* __restrict__ nlist,
     unsigned int* __restrict__ n_neigh, BCond* __restrict__ cond)
 {
 #pragma clang fp contract(off)
@@ -479,7 +482,7 @@ __global__ __launch_bounds__(64 * NL_WAVES) void bnlist_kernel(
             const float hy = rel ? centre_offset(xi.y, ccy, R) : 0.f;
             const float hz = rel ? centre_offset(xi.z, ccz, R) : 0.f;
             unsigned int cnt = hcnt[h];
-            unsigned int* row = nlist + (size_t)i * nmax;
+            unsigned int* row = nlist + (size_t)i * stride;
             for (unsigned int k0 = 0; k0 < npass; k0 += 64)
             {
                 const unsigned int k = k0 + lane;
@@ -505,7 +508,7 @@ __global__ __launch_bounds__(64 * NL_WAVES) void bnlist_kernel(
                 const uint64_t m = wave_ballot(hit);
                 const unsigned int at = cnt + lanes_below(m);
                 if (hit && at < nmax)
-                    row[at] = e;
+                    row[row_store_pos(at)] = e;
                 cnt += (unsigned int)__popcll(m);
             }
             if (lane == 0)
@@ -541,15 +544,28 @@ __device__ __forceinline__ void lj_accumulate(const PairConst& pc, float rsq, fl
     fz += dz * fdr;
 }
 
+// Rows are in transposed blocks of ROW_BLOCK entries (row_store_pos): a lane reads four entries with one
+// 16-byte load, and for each of the four the lanes of a particle hold consecutive neighbours. The cell
+// offset of an entry comes from a table in LDS. Workgroups are in XCD order, so a replica's particles
+// stay in one L2. 1.3e6 particles in 256 replicas, 105e6 entries: 210 us a launch, before 218 (4-byte row
+// loads, the offset decoded by divisions: 25 vector instructions of a pair's 60).
 template<unsigned int TPP>
 __global__ __launch_bounds__(256) void bpair_kernel(
     const Rep* __restrict__ reps, const unsigned int* __restrict__ part_rep, unsigned int N,
     const double4* __restrict__ pos, const unsigned int* __restrict__ nlist, unsigned int nmax,
-    const unsigned int* __restrict__ n_neigh, PairConst pc, float4* __restrict__ force,
-    const float4* __restrict__ rel)
+    unsigned int stride, const unsigned int* __restrict__ n_neigh, PairConst pc,
+    float4* __restrict__ force, const float4* __restrict__ rel)
 {
 #pragma clang fp contract(off)
-    const unsigned int g = blockIdx.x * blockDim.x + threadIdx.x;
+    __shared__ float4 offset[32];
+    if (threadIdx.x < 32)
+    {
+        const unsigned int c = threadIdx.x;
+        offset[c] = make_float4((float)((int)(c % 3u) - 1), (float)((int)((c / 3u) % 3u) - 1),
+                                (float)((int)(c / 9u) - 1), 0.f);
+    }
+    __syncthreads();
+    const unsigned int g = xcd_block(blockIdx.x, gridDim.x) * blockDim.x + threadIdx.x;
     const unsigned int p = g / TPP;
     const unsigned int sub = g % TPP;
     float fx = 0.f, fy = 0.f, fz = 0.f, e = 0.f;
@@ -561,45 +577,39 @@ __global__ __launch_bounds__(256) void bpair_kernel(
         const float w = (float)R.w;
         const float guard = pc.guard_w * w + pc.guard_0;
         const unsigned int nn = min(n_neigh[p], nmax);
-        const unsigned int* row = nlist + (size_t)p * nmax;
-        for (unsigned int k0 = sub; k0 < nn; k0 += TPP * UNR)
+        const uint4* row4 = (const uint4*)(nlist + (size_t)p * stride);
+        for (unsigned int k0 = 0; k0 < ((nn + ROW_BLOCK - 1) & ~(ROW_BLOCK - 1)); k0 += TPP * UNR)
         {
-            unsigned int en[UNR];
-#pragma unroll
-            for (unsigned int u = 0; u < UNR; u++)
-            {
-                const unsigned int k = k0 + u * TPP;
-                // the particle itself, at zero offset, stands in for missing entries
-                en[u] = k < nn ? row[k] : (p | (BCODE_SELF << BCODE_SHIFT));
-            }
+            // entries past the row's count are valid indices of an older list (rows are followed by
+            // NLIST_PAD zeros) and are masked
+            const uint4 v = row4[(k0 >> 2) + sub];
+            const unsigned int en[UNR] = {v.x, v.y, v.z, v.w};
             float4 rj[UNR];
 #pragma unroll
             for (unsigned int u = 0; u < UNR; u++)
-                rj[u] = rel[en[u] & BJ_MASK];
+                rj[u] = rel[min(en[u] & BJ_MASK, N - 1)];
 #pragma unroll
             for (unsigned int u = 0; u < UNR; u++)
             {
-                const unsigned int j = en[u] & BJ_MASK, code = en[u] >> BCODE_SHIFT;
-                const float ox = (float)((int)(code % 3u) - 1);
-                const float oy = (float)((int)((code / 3u) % 3u) - 1);
-                const float oz = (float)((int)(code / 9u) - 1);
-                const float dx = (ri.x - rj[u].x) - ox * w;
-                const float dy = (ri.y - rj[u].y) - oy * w;
-                const float dz = (ri.z - rj[u].z) - oz * w;
+                const bool valid = row_neighbour(k0 + 4u * sub + u) < nn;
+                const float4 o = offset[en[u] >> BCODE_SHIFT & 31u];
+                const float dx = (ri.x - rj[u].x) - o.x * w;
+                const float dy = (ri.y - rj[u].y) - o.y * w;
+                const float dz = (ri.z - rj[u].z) - o.z * w;
                 const float rsq = dx * dx + dy * dy + dz * dz;
                 const float t = rsq - pc.rcutsq_f;
-                bool in = t < 0.f;
-                if (fabsf(t) <= guard)
+                bool in = valid && t < 0.f;
+                if (valid && fabsf(t) <= guard)
                 {
                     // exact FP64 decision (the FP64 form of this kernel)
-                    const double4 xi = pos[p], xj = pos[j];
+                    const double4 xi = pos[p], xj = pos[en[u] & BJ_MASK];
                     double ddx = xi.x - xj.x, ddy = xi.y - xj.y, ddz = xi.z - xj.z;
                     ddz -= R.L * rint(ddz * R.Linv);
                     ddy -= R.L * rint(ddy * R.Linv);
                     ddx -= R.L * rint(ddx * R.Linv);
                     in = ddx * ddx + ddy * ddy + ddz * ddz < pc.rcutsq;
                 }
-                if (in && j != p)
+                if (in)
                     lj_accumulate(pc, rsq, dx, dy, dz, fx, fy, fz, e);
             }
         }
@@ -609,7 +619,7 @@ __global__ __launch_bounds__(256) void bpair_kernel(
         const Rep R = reps[part_rep[p]];
         const double4 xi = pos[p];
         const unsigned int nn = min(n_neigh[p], nmax);
-        const unsigned int* row = nlist + (size_t)p * nmax;
+        const unsigned int* row = nlist + (size_t)p * stride;
         // UNR neighbours per lane per pass: every index, then every position load is issued
         // before the first is used, so several gathers are in flight per lane
         for (unsigned int k0 = sub; k0 < nn; k0 += TPP * UNR)
@@ -619,7 +629,7 @@ __global__ __launch_bounds__(256) void bpair_kernel(
             for (unsigned int u = 0; u < UNR; u++)
             {
                 const unsigned int k = k0 + u * TPP;
-                j[u] = k < nn ? row[k] : p;
+                j[u] = k < nn ? row[row_store_pos(k)] : p;
             }
             double4 xj[UNR];
 #pragma unroll
@@ -693,6 +703,48 @@ __global__ __launch_bounds__(BTILE) void bstep_two_kernel(
     }
 }
 
+// -------------------------------------------------------------------------- reading the state
+// Particles sit in cell order; particle n was created at its replica's offset plus its tag. The packed
+// arrays leave the device in that order, where the host once copied the padded ones and reordered them
+// (34 ms for 1.3e6 particles, most of 100 steps; 6 ms now).
+__device__ __forceinline__ size_t created_at(const Rep* reps, const unsigned int* part_rep,
+                                             const unsigned int* tag, unsigned int n)
+{
+    return (size_t)reps[part_rep[n]].off + tag[n];
+}
+
+__global__ __launch_bounds__(256) void bread_vec_kernel(const Rep* __restrict__ reps,
+                                                        const unsigned int* __restrict__ part_rep,
+                                                        const unsigned int* __restrict__ tag,
+                                                        unsigned int N, const double4* __restrict__ v,
+                                                        double* __restrict__ out)
+{
+    const unsigned int n = blockIdx.x * 256u + threadIdx.x;
+    if (n >= N)
+        return;
+    const size_t i = created_at(reps, part_rep, tag, n);
+    const double4 x = v[n];
+    out[3 * i] = x.x;
+    out[3 * i + 1] = x.y;
+    out[3 * i + 2] = x.z;
+}
+
+__global__ __launch_bounds__(256) void bread_image_kernel(const Rep* __restrict__ reps,
+                                                          const unsigned int* __restrict__ part_rep,
+                                                          const unsigned int* __restrict__ tag,
+                                                          unsigned int N, const i3* __restrict__ v,
+                                                          int* __restrict__ out)
+{
+    const unsigned int n = blockIdx.x * 256u + threadIdx.x;
+    if (n >= N)
+        return;
+    const size_t i = created_at(reps, part_rep, tag, n);
+    const i3 x = v[n];
+    out[3 * i] = x.x;
+    out[3 * i + 1] = x.y;
+    out[3 * i + 2] = x.z;
+}
+
 // -------------------------------------------------------------------------- cell order
 // The particles of each replica re-laid in cell order (cells in index order, each cell's
 // particles by index), so that the particles a wavefront gathers in the list build and the pair
@@ -757,6 +809,8 @@ struct hm_batch
     double dt = 0.005, tau = 0.0, r_cut = 2.5, r_buff = 0.4, rlistsq = 0.0, maxsq = 0.0;
     PairConst pc{};
     unsigned int cmax = 0, nmax = 0;
+    // row length in memory: whole transposed blocks
+    unsigned int stride() const { return round_up(nmax, ROW_BLOCK); }
     unsigned int pair_tpp = 4, pair_block = 256;
     bool tuned = false;
     unsigned int chunk = 100;
@@ -844,9 +898,9 @@ struct hm_batch
         bfree(nlist);
         cell_raw = balloc<unsigned int>((size_t)ncell * cmax);
         cell_idx = balloc<unsigned int>((size_t)ncell * cmax);
-        nlist = balloc<unsigned int>((size_t)N * nmax);
+        nlist = balloc<unsigned int>((size_t)N * stride() + NLIST_PAD);
         // zero-filled: every row entry and count is a valid index / length before any build
-        bchk(hipMemset(nlist, 0, sizeof(unsigned int) * (size_t)N * nmax), "clear rows");
+        bchk(hipMemset(nlist, 0, sizeof(unsigned int) * ((size_t)N * stride() + NLIST_PAD)), "clear rows");
         bchk(hipMemset(cell_idx, 0, sizeof(unsigned int) * (size_t)ncell * cmax), "clear cells");
         if (n_neigh)
             bchk(hipMemset(n_neigh, 0, sizeof(unsigned int) * N), "clear counts");
@@ -857,28 +911,28 @@ struct hm_batch
     void launch_pair()
     {
         const unsigned int nthreads = N * pair_tpp;
-        const dim3 grid((nthreads + pair_block - 1) / pair_block), block(pair_block);
+        const dim3 grid(round_up((nthreads + pair_block - 1) / pair_block, 8)), block(pair_block);
         switch (pair_tpp)
         {
         case 1:
             hipLaunchKernelGGL(bpair_kernel<1>, grid, block, 0, stream, reps, part_rep, N, pos,
-                               nlist, nmax, n_neigh, pc, force, rel);
+                               nlist, nmax, stride(), n_neigh, pc, force, rel);
             break;
         case 2:
             hipLaunchKernelGGL(bpair_kernel<2>, grid, block, 0, stream, reps, part_rep, N, pos,
-                               nlist, nmax, n_neigh, pc, force, rel);
+                               nlist, nmax, stride(), n_neigh, pc, force, rel);
             break;
         case 4:
             hipLaunchKernelGGL(bpair_kernel<4>, grid, block, 0, stream, reps, part_rep, N, pos,
-                               nlist, nmax, n_neigh, pc, force, rel);
+                               nlist, nmax, stride(), n_neigh, pc, force, rel);
             break;
         case 8:
             hipLaunchKernelGGL(bpair_kernel<8>, grid, block, 0, stream, reps, part_rep, N, pos,
-                               nlist, nmax, n_neigh, pc, force, rel);
+                               nlist, nmax, stride(), n_neigh, pc, force, rel);
             break;
         default:
             hipLaunchKernelGGL(bpair_kernel<16>, grid, block, 0, stream, reps, part_rep, N, pos,
-                               nlist, nmax, n_neigh, pc, force, rel);
+                               nlist, nmax, stride(), n_neigh, pc, force, rel);
             break;
         }
         bchk(hipGetLastError(), "batch pair");
@@ -895,7 +949,7 @@ struct hm_batch
                            0, stream, cell_rep, rst, ncell, cmax, cell_size, cell_raw, cell_idx);
         hipLaunchKernelGGL(bnlist_kernel, dim3(ncell), dim3(64 * NL_WAVES), 0, stream, reps,
                            cell_rep, rst,
-                           pos, cmax, cell_size, cell_idx, rlistsq, nmax, nlist, n_neigh, cond);
+                           pos, cmax, cell_size, cell_idx, rlistsq, nmax, stride(), nlist, n_neigh, cond);
         bchk(hipGetLastError(), "batch rebuild");
     }
 
@@ -1014,6 +1068,12 @@ struct hm_batch
         return K;
     }
 
+    void reserve_stage()
+    {
+        if (!stage)
+            stage = balloc<double4>(N);
+    }
+
     // Re-lay every replica's particles in cell order (between chunks, outside any graph): a
     // fresh binning of all replicas, the per-replica cell starts, the order, the permutation of
     // every per-particle array, then the kinetic-energy partials of the new tiles and a forced
@@ -1024,7 +1084,7 @@ struct hm_batch
         {
             cell_start = balloc<unsigned int>(ncell);
             order = balloc<unsigned int>(N);
-            stage = balloc<double4>(N);
+            reserve_stage();
         }
         for (int attempt = 0;; attempt++)
         {
@@ -1555,36 +1615,35 @@ int hm_batch_get_state(hm_batch* b, double* pos3, double* vel3, int* image3)
     if (!b)
         return fail(HM_ERR_ARGS, "hm_batch_get_state: NULL batch");
     return bguard([&]() {
-        const unsigned int N = b->N;
-        std::vector<double4> p(N), v(N);
-        std::vector<i3> im(N);
-        bchk(hipStreamSynchronize(b->stream), "sync");
-        bchk(hipMemcpy(p.data(), b->pos, sizeof(double4) * N, hipMemcpyDeviceToHost), "pos");
-        bchk(hipMemcpy(v.data(), b->vel, sizeof(double4) * N, hipMemcpyDeviceToHost), "vel");
-        bchk(hipMemcpy(im.data(), b->image, sizeof(i3) * N, hipMemcpyDeviceToHost), "image");
-        const std::vector<unsigned int> where = b->creation_index();
-        for (unsigned int n = 0; n < N; n++)
+        const size_t words = (size_t)3 * b->N;
+        b->reserve_stage();
+        double* const packed = (double*)b->stage;  // the sort's scratch: 32 bytes per particle
+        // each array is put into the order of creation on the device and copied straight out
+        auto copy_out = [&](void* dst, size_t bytes) {
+            bchk(hipGetLastError(), "state order");
+            bchk(hipMemcpyAsync(dst, packed, bytes, hipMemcpyDeviceToHost, b->stream), "state");
+            bchk(hipStreamSynchronize(b->stream), "sync");
+        };
+        const dim3 grid((b->N + 255) / 256), block(256);
+        if (pos3)
         {
-            const unsigned int i = where[n];
-            if (pos3)
-            {
-                pos3[3 * i] = p[n].x;
-                pos3[3 * i + 1] = p[n].y;
-                pos3[3 * i + 2] = p[n].z;
-            }
-            if (vel3)
-            {
-                vel3[3 * i] = v[n].x;
-                vel3[3 * i + 1] = v[n].y;
-                vel3[3 * i + 2] = v[n].z;
-            }
-            if (image3)
-            {
-                image3[3 * i] = im[n].x;
-                image3[3 * i + 1] = im[n].y;
-                image3[3 * i + 2] = im[n].z;
-            }
+            hipLaunchKernelGGL(bread_vec_kernel, grid, block, 0, b->stream, b->reps, b->part_rep,
+                               b->tag, b->N, b->pos, packed);
+            copy_out(pos3, words * sizeof(double));
         }
+        if (vel3)
+        {
+            hipLaunchKernelGGL(bread_vec_kernel, grid, block, 0, b->stream, b->reps, b->part_rep,
+                               b->tag, b->N, b->vel, packed);
+            copy_out(vel3, words * sizeof(double));
+        }
+        if (image3)
+        {
+            hipLaunchKernelGGL(bread_image_kernel, grid, block, 0, b->stream, b->reps, b->part_rep,
+                               b->tag, b->N, b->image, (int*)packed);
+            copy_out(image3, words * sizeof(int));
+        }
+        bchk(hipStreamSynchronize(b->stream), "sync");
         return HM_OK;
     });
 }

@@ -102,4 +102,31 @@ __device__ __forceinline__ void count_build(const NlistKernelArgs& a)
     }
 }
 
+// The next slot of cell bin for every lane with ok, called by every lane of a wavefront in step; the
+// active lanes must be its low lanes.
+__device__ __forceinline__ unsigned int claim_slot(unsigned int bin, bool ok, unsigned int* cell_size)
+{
+    // slot allocation aggregated over runs of consecutive lanes in one cell (particles in
+    // Hilbert order fill a cell from neighbouring indices): the first lane of a run adds the
+    // run's length, and every run's atomic is issued by the one instruction. Active lanes are
+    // the low lanes of the wave, so a lane's predecessor is active.
+    const unsigned int lane = lane_id();
+    const unsigned int prev = __shfl_up(bin, 1, 64);
+    const bool head = ok && (lane == 0 || prev != bin || !__shfl_up((int)ok, 1, 64));
+    const uint64_t heads = wave_ballot(head);
+    // lanes that do not continue a run: heads, lanes not binned, inactive lanes
+    const uint64_t stop = ~wave_ballot(ok && !head);
+    const uint64_t upto = lane == 63 ? ~0ull : ((1ull << (lane + 1)) - 1ull);
+    const unsigned int first = 63u - (unsigned int)__clzll((long long)(heads & upto));
+    unsigned int base = 0;
+    if (head)
+    {
+        const uint64_t after = lane == 63 ? 0ull : (stop >> (lane + 1));
+        const unsigned int len = after ? (unsigned int)__ffsll((long long)after) : 64u - lane;
+        base = atomicAdd(&cell_size[bin], len);
+    }
+    base = __shfl(base, (int)(ok ? first : lane), 64);
+    return ok ? base + (lane - first) : 0u;
+}
+
 } // namespace hm

@@ -117,27 +117,7 @@ __device__ __forceinline__ void bin_particle(unsigned int n, const double4* __re
             else
                 bin = (unsigned int)((kb * (int)dy + jb) * (int)dx + ib);
         }
-        // slot allocation aggregated over runs of consecutive lanes in one cell (particles in
-        // Hilbert order fill a cell from neighbouring indices): the first lane of a run adds the
-        // run's length, and every run's atomic is issued by the one instruction. Active lanes are
-        // the low lanes of the wave, so a lane's predecessor is active.
-        const unsigned int lane = lane_id();
-        const unsigned int prev = __shfl_up(bin, 1, 64);
-        const bool head = ok && (lane == 0 || prev != bin || !__shfl_up((int)ok, 1, 64));
-        const uint64_t heads = wave_ballot(head);
-        // lanes that do not continue a run: heads, lanes not binned, inactive lanes
-        const uint64_t stop = ~wave_ballot(ok && !head);
-        const uint64_t upto = lane == 63 ? ~0ull : ((1ull << (lane + 1)) - 1ull);
-        const unsigned int first = 63u - (unsigned int)__clzll((long long)(heads & upto));
-        unsigned int base = 0;
-        if (head)
-        {
-            const uint64_t after = lane == 63 ? 0ull : (stop >> (lane + 1));
-            const unsigned int len = after ? (unsigned int)__ffsll((long long)after) : 64u - lane;
-            base = atomicAdd(&cell_size[bin], len);
-        }
-        base = __shfl(base, (int)(ok ? first : lane), 64);
-        const unsigned int slot = ok ? base + (lane - first) : 0u;
+        const unsigned int slot = claim_slot(bin, ok, cell_size);
         const bool placed = ok && slot < cmax;
         if (ok && !placed)
             atomicMax(&cond[0], slot + 1);

@@ -138,3 +138,64 @@ def test_tuner_and_long_run(B):
     b2 = B.ReplicaBatch(pos, L, kT, seeds)
     b2.thermalize(0)
     assert len(b2.tune()) == 0 and b2.config["tpp"] == b.config["tpp"]
+
+
+def row_fluids(B):
+    """Boxes of two cells an axis (FP64 rows) and of three to five, with rows that end anywhere in
+    their last block of entries."""
+    rng = np.random.default_rng(5)
+    n = [180, 521, 1100, 2817]
+    L = [(k / r) ** (1.0 / 3.0) for k, r in zip(n, (0.7, 0.85, 0.75, 0.9))]
+    return L, [B.fcc_fill(k, e, rng) for k, e in zip(n, L)]
+
+
+def pair_magnitudes(L, x):
+    """Per particle the sums of |f| and of the magnitudes of the two terms of the halved energy."""
+    size, esize = np.zeros(len(x)), np.zeros(len(x))
+    for i in range(len(x)):
+        d = x[i] - x
+        d -= L * np.rint(d / L)
+        r2 = (d * d).sum(1)
+        r2 = r2[(r2 > 0) & (r2 < 6.25)]
+        i6 = r2 ** -3.0
+        size[i] = (np.abs(48 * i6 * i6 - 24 * i6) / np.sqrt(r2)).sum()
+        esize[i] = 2 * (i6 * i6 + i6).sum()
+    return size, esize
+
+
+@pytest.mark.parametrize("tpp,block", [(1, 64), (2, 128), (4, 256), (8, 64), (16, 256)])
+def test_every_pair_launch_sums_the_whole_rows(B, tpp, block):
+    L, pos = row_fluids(B)
+    b = B.ReplicaBatch(pos, L, [1.0] * 4, [1, 2, 3, 4])
+    b.set_pair_launch(tpp, block)
+    forces = b.forces()
+    for r in range(4):
+        nl, nn = O.nlist_binned(O.Box(L[r]), pos[r], 2.5, 0.4, full=True)
+        rf, _ = O.pair_lj(O.Box(L[r]), pos[r], nl, nn, third_law=False)
+        # the lattice's pair forces cancel, so the bound is on their magnitudes: a pair force r^-13
+        # turns the rounding of an FP32 separation (under 4 ulp of a 3 sigma cell, r > 0.9) into 13 *
+        # 4 * 3 / 0.9 < 180 units of 2^-24, its arithmetic and a sum of 60 terms add fewer than 76
+        size, esize = pair_magnitudes(L[r], pos[r])
+        assert (np.linalg.norm(forces[r][:, :3] - rf[:, :3], axis=1) <= 256 * 2.0 ** -24 * size).all()
+        assert (np.abs(forces[r][:, 3] - rf[:, 3]) <= 256 * 2.0 ** -24 * esize).all()
+
+
+def test_state_comes_back_in_creation_order(B):
+    """Sorted before every step and never sorted: the same particles in the same places. Ten steps
+    part the two by the rounding of the FP32 force sums (1e-5 relative, as the trajectories' bar)."""
+    L, pos = row_fluids(B)
+    got = []
+    for period in (0, 1):
+        b = B.ReplicaBatch(pos, L, [1.0] * 4, [1, 2, 3, 4], sort_period=period)
+        b.thermalize(0)
+        x0, v0, im0 = b.state()
+        assert all(np.array_equal(x0[r], pos[r]) and (im0[r] == 0).all() for r in range(4))
+        for _ in range(10):
+            b.run(1)
+        got.append((b.state(), v0))
+    for r in range(4):
+        (xa, va, ia), v0 = [q[r] for q in got[0][0]], got[0][1][r]
+        xb, vb, ib = [q[r] for q in got[1][0]]
+        assert np.array_equal(v0, got[1][1][r])
+        ua, ub = xa + ia * L[r], xb + ib * L[r]
+        assert np.abs(ua - ub).max() < 1e-5 and rel_rms(vb - v0, va - v0) < 1e-5
