@@ -58,11 +58,12 @@ __device__ __forceinline__ unsigned int wave_prefix(unsigned int v, unsigned int
     return v;
 }
 
-// One neighbour test shifted into the low end of mask m: bit = (t <= 0). One compare and one
-// add-with-carry, which the compiler does not form from the shift and the or by itself.
+// One neighbour test shifted into the low end of mask m: the sign of t. A t of zero, whose sign says
+// nothing, lies in every guard band. One v_alignbit; a compare into VCC and an add with carry would need
+// two wait states between them on gfx950.
 __device__ __forceinline__ void push_hit(unsigned int& m, float t)
 {
-    asm("v_cmp_ge_f32 vcc, 0, %1\n\tv_addc_co_u32 %0, vcc, %0, %0, vcc" : "+v"(m) : "v"(t) : "vcc");
+    m = __builtin_amdgcn_alignbit(m, __float_as_uint(t), 31);
 }
 
 // place (0, 1, 2) of offset o among the neighbours h - 1, h, h + 1 sorted by wrapped coordinate; rank is
