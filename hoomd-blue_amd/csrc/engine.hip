@@ -245,6 +245,11 @@ struct hm_system
     // list-build launch shape (0: from the occupancy) and persistent grid, from the autotuner
     int nl_shape = 0;
     unsigned int nl_grid = 0;
+    bool nl_fixed = false;            // set by the caller: not swept
+    // The sweep takes columns on the state it sees. Where a twentieth of the particles has come to lie in
+    // columns that do not fit their stage (a fluid that condenses; a choice from the cache), both forms
+    // are timed again, once: such a particle's row costs about seven times a staged one.
+    bool crowd_seen = false, crowd_tuned = false;
     // second sweep once the system has run this many steps since its first prep (the lattice
     // start is more ordered than the liquid it melts into)
     uint64_t retune_after = 500;
@@ -565,6 +570,7 @@ struct hm_system
         k.check_delay = check_delay;
         k.dist_check = dist_check;
         k.slot_of = slot_of;
+        k.crowded = &cond->crowded;
         if (uses_rel())
         {
             // the cell ordering of this build wrote the relative positions the list stages
@@ -1111,17 +1117,16 @@ struct hm_system
     void tune_nlist()
     {
         nl_log.clear();
+        if (nl_fixed)
+            return;
         if (rcut_max <= 0.0 || !nlist)
             return;
-        {
-            NlistKernelArgs k;
-            fill_nlist_args(k, false);
-            if (nlist_uses_columns(k))
-                return;  // one launch shape
-        }
+        const bool columns = columns_apply();
         std::vector<int> shapes{0};
         if (cmax <= 64)
             shapes = {NL_SHAPE_TINY, NL_SHAPE_SMALL, NL_SHAPE_MID, NL_SHAPE_BIG};
+        if (columns)
+            shapes.push_back(NL_SHAPE_COLUMNS);
         hipEvent_t ev[4];
         for (auto& e : ev)
             hchk(hipEventCreate(&e), "event");
@@ -1134,6 +1139,8 @@ struct hm_system
             std::vector<unsigned int> grids =
                 one_wave ? std::vector<unsigned int>{2048u, 4096u, 8192u, 16384u}
                          : std::vector<unsigned int>{1024u, 2048u, 4096u, 8192u};
+            if (sh == NL_SHAPE_COLUMNS)
+                grids = {0u};  // from its geometry
             // one-wavefront shapes also try one workgroup per cell (no persistent loop)
             if (one_wave && round_up(ncell, 8) > 16384u)
                 grids.push_back(round_up(ncell, 8));
@@ -1176,6 +1183,17 @@ struct hm_system
         clear_graphs();
     }
 
+    // whether the present list could be built over columns of cells
+    bool columns_apply()
+    {
+        if (rcut_max <= 0.0 || !nlist)
+            return false;
+        NlistKernelArgs k;
+        fill_nlist_args(k, false);
+        k.shape = NL_SHAPE_COLUMNS;
+        return nlist_uses_columns(k);
+    }
+
     // the whole sweep: the shape cache (same kind of system seen before in this process), else
     // the list build then the pair kernel, and the result stored in the cache
     void tune_all(bool use_cache)
@@ -1186,8 +1204,11 @@ struct hm_system
         {
             const TuneChoice& c = it->second;
             pair_launch_cfg() = c.pair;
-            nl_shape = c.nl_shape;
-            nl_grid = c.nl_grid;
+            if (!nl_fixed)
+            {
+                nl_shape = c.nl_shape;
+                nl_grid = c.nl_grid;
+            }
             pair_tuned = true;
             tune_cached = true;
             tune_log.clear();
@@ -1198,7 +1219,8 @@ struct hm_system
         tune_cached = false;
         tune_nlist();
         tune_pair();
-        g_tune_cache()[key] = TuneChoice{pair_launch_cfg(), nl_shape, nl_grid};
+        if (!nl_fixed)
+            g_tune_cache()[key] = TuneChoice{pair_launch_cfg(), nl_shape, nl_grid};
     }
 
     PairLaunch& pair_launch_cfg()
@@ -1209,7 +1231,7 @@ struct hm_system
 
     // bucket of systems that share launch shapes: pair kind, force kinds, types, exclusions,
     // log2 N in half steps, density, list range and cells per axis (coarse)
-    std::string tune_key() const
+    std::string tune_key()
     {
         const double vol = hbox.L[0] * hbox.L[1] * hbox.L[2];
         char buf[256];
@@ -1529,8 +1551,16 @@ struct hm_system
                 if (rcut_max > 0.0)
                     build_nlist_now();
                 tune_all(false);
+                crowd_seen = false;
                 // the sweep's list builds reused the last cell binning: rebuild both before the
                 // forces of the next step
+                hchk(launch_set_rebuild(st, stream), "force rebuild");
+            }
+            if (crowd_seen && !crowd_tuned && !nl_fixed)
+            {
+                crowd_tuned = true;
+                build_nlist_now();
+                tune_nlist();
                 hchk(launch_set_rebuild(st, stream), "force rebuild");
             }
             if (sort_period && timestep % sort_period == 0 && last_sort_step != timestep)
@@ -1574,6 +1604,8 @@ struct hm_system
                 throw HmError{HM_ERR_THERMO, "Bussi thermostat requires non-zero initial momenta"};
             }
             retries = 0;
+            const uint64_t built = s.n_builds - s_state.n_builds;
+            crowd_seen = crowd_seen || (built > 0 && c.crowded > built * N / 20);
             timestep += K;
             steps_run += K;
         }
@@ -2073,6 +2105,19 @@ int hm_sys_tune_log(const hm_system* s, float* out, unsigned int max_rows)
 void hm_tune_cache_clear(void)
 {
     g_tune_cache().clear();
+}
+
+int hm_sys_set_nlist_launch(hm_system* s, int shape, unsigned int grid)
+{
+    if (!s || shape < 0 || shape > NL_SHAPE_COLUMNS || grid > 65536)
+        return fail(HM_ERR_ARGS, "hm_sys_set_nlist_launch: invalid arguments");
+    s->nl_shape = shape;
+    s->nl_grid = grid;
+    s->nl_fixed = shape != 0;
+    s->pair_tuned = s->pair_tuned && s->nl_fixed;  // 0: swept again at the next run
+    s->prepared = s->configured = false;
+    s->clear_graphs();
+    return HM_OK;
 }
 
 int hm_sys_nlist_launch(const hm_system* s, int out[3], float* log3, unsigned int max_rows)

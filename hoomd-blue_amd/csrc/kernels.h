@@ -54,7 +54,8 @@ struct Conditions
     unsigned int out_idx;     // particle + 1
     unsigned int nlist_need;  // required nmax
     unsigned int bond_flag;
-    unsigned int pad[3];
+    unsigned int crowded;     // particles of columns that did not fit their stage, over all builds
+    unsigned int pad[2];
 };
 
 struct PairLaunch
@@ -198,10 +199,12 @@ struct NlistKernelArgs
     const float3* srel;
     const unsigned int* sidx;
     const uint32_t* swrd;
-    const uint32_t* slot_of;  // slot of each particle (exclusions of rows with offset codes)
+    const uint32_t* slot_of;  // slot of each particle (exclusions of the column build)
+    unsigned int* crowded;    // Conditions::crowded, or NULL
     float cwf[3];             // cell widths rounded to FP32
     // launch shape, 0 = chosen from the cell occupancy. shape: workgroup form of the FP32 path
-    // (NL_SHAPE_*; a form whose home-cell capacity is below cmax falls back to the default);
+    // (NL_SHAPE_*; a form whose home-cell capacity is below cmax falls back to the default, and so do
+    // columns where they do not apply);
     // grid: persistent workgroups (rounded up to a multiple of 8)
     int shape;
     unsigned int grid;
@@ -212,6 +215,7 @@ enum : int
     NL_SHAPE_SMALL = 2,
     NL_SHAPE_MID = 3,
     NL_SHAPE_BIG = 4,
+    NL_SHAPE_COLUMNS = 5,
 };
 
 // Cell-tiled pair kernel: neighbours read from the home cell's LDS-staged candidates through
@@ -267,7 +271,7 @@ hipError_t launch_cell_bin_rank(unsigned int N, const unsigned int dim[3], unsig
                                 const StepState* gate, hipStream_t s, const DevBox& box,
                                 const RelFrame& rel);
 hipError_t launch_nlist_build(const NlistKernelArgs& a, hipStream_t s);
-// whether that launch builds over columns of cells (its shape and grid are then not used)
+// whether that launch builds over columns of cells (shape NL_SHAPE_COLUMNS; its grid is then not used)
 bool nlist_uses_columns(const NlistKernelArgs& a);
 
 hipError_t launch_nlist_check(unsigned int N, const double4* pos, const d3* last,

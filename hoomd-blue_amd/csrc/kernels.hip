@@ -970,17 +970,20 @@ static void nlist_dispatch(const NlistKernelArgs& a, bool mt, bool ex, unsigned 
                            a);
 }
 
-// Cells of a few particles are built over columns (tile.hip). Index rows, us a build, cell form below ->
-// columns: 10^6 particles, 3.0 a cell 405 -> 254, 6.7 a cell 397 -> 302; 131 072, 3.1 a cell 58 -> 38,
-// 7.5 a cell 59 -> 43; 50 021, 3.2 a cell 27 -> 22, 7.3 a cell 28 -> 24; at 16 384 the two are equal
-// (15 -> 16), and at 21 a cell the cell form's wavefront per home particle is the better one (520
-// against 606 at 10^6). The cell form also keeps the 16-bit local rows, grids with fewer than 4
-// cells along an axis, and exclusions given without the slot of each particle.
+// Where cells hold a few particles the list can be built over columns (tile.hip). Index rows, us a build,
+// cell form below -> columns: 10^6 particles, 3.0 a cell 405 -> 254, 6.7 a cell 397 -> 302; 131 072, 3.1 a
+// cell 58 -> 38, 7.5 a cell 59 -> 43; 50 021, 3.2 a cell 27 -> 22, 7.3 a cell 28 -> 24; at 16 384 the two are
+// equal (15 -> 16), and at 21 a cell the cell form's wavefront per home particle is the better one (520
+// against 606 at 10^6). These are uniform fluids. A slab of 20 a cell beside vapour (33 000 particles, 6.7 on
+// the mean) takes 248 us over columns and 37 in the cell form, which the mean does not tell: columns are
+// built only where the caller asks for them, as the engine does after timing both. The cell form also keeps
+// the 16-bit local rows, grids with fewer than 4 cells along an axis, and exclusions given without the slot
+// of each particle.
 constexpr unsigned int COL_MIN_N = 32768;
 
 static bool column_build_applies(const NlistKernelArgs& a, ColGeom& g)
 {
-    return a.pos && (a.entries || a.srel) && !a.lrow && !a.skip_index_rows && a.n_adj == 27
+    return a.shape == NL_SHAPE_COLUMNS && a.pos && (a.entries || a.srel) && !a.lrow && !a.skip_index_rows && a.n_adj == 27
            && (!a.offset_codes || a.sidx) && (!a.n_excl || a.max_excl == 0 || a.slot_of)
            && a.N >= COL_MIN_N && a.N <= 8ull * a.ncell && choose_columns(a.N, a.dim, g);
 }
@@ -1008,7 +1011,7 @@ hipError_t launch_nlist_build(const NlistKernelArgs& a_in, hipStream_t s)
     // an explicit shape (the autotuner's) where its home-cell capacity holds cmax; the staging
     // passes of every shape take any number of candidates
     bool mid_ok = a.cmax <= (unsigned int)NlMid::HOME;
-    if (a.shape && a.cmax <= (unsigned int)NlSmall::HOME)
+    if (a.shape && a.shape != NL_SHAPE_COLUMNS && a.cmax <= (unsigned int)NlSmall::HOME)
     {
         tiny = a.shape == NL_SHAPE_TINY;
         small = tiny || a.shape == NL_SHAPE_SMALL;

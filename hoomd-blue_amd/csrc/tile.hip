@@ -235,6 +235,8 @@ __global__ __launch_bounds__(COL_BLOCK) void nlist_col_kernel(NlistKernelArgs a,
         __syncthreads();
         const unsigned int total = S.off[nsc], nhome = S.hoff[nh];
         const bool fits = total <= g.cap && nhome <= g.hcap;
+        if (!fits && a.crowded && tid == 0)
+            atomicAdd(a.crowded, nhome);
         if (fits)
             for (unsigned int q = sgrp; q < nsc; q += nsgrp)
             {

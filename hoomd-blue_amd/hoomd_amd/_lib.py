@@ -190,6 +190,7 @@ SIGNATURES = {
     "hm_sys_time_mlp": (_i, [_p, _i, _u, _p]),
     "hm_sys_time_build": (_i, [_p, _u, _p]),
     "hm_sys_set_list_capacity": (_i, [_p, _u, _u]),
+    "hm_sys_set_nlist_launch": (_i, [_p, _i, _u]),
     "hm_sys_nlist_launch": (_i, [_p, _p, _p, _u]),
     "hm_tune_cache_clear": (None, []),
     "hm_sys_frame_subtract_force": (_i, [_p, _i, _p, _p]),

@@ -481,12 +481,17 @@ int hm_sys_pair_config(const hm_system* s, unsigned int out[5]);
 /* Autotuner samples of the last sweep: rows of (tpp, size, batch, median ms), at most max_rows
  * written; returns the number of rows of the sweep. */
 int hm_sys_tune_log(const hm_system* s, float* out, unsigned int max_rows);
+/* List-build launch: shape and grid as in hm_sys_nlist_launch; a shape other than 0 is kept and not swept,
+ * 0 gives the choice back to the autotuner. A shape that does not apply to the system's cells builds
+ * in the default one. */
+int hm_sys_set_nlist_launch(hm_system* s, int shape, unsigned int grid);
 /* List-build launch chosen by the autotuner: out[0] = workgroup shape (0 default, 1 tiny,
- * 2 small, 3 mid, 4 big), out[1] = persistent grid (0 default), out[2] = 1 when the choice came
- * from the process's cache of earlier sweeps (same pair kind, forces, types, exclusions, size,
- * density, list range and cell grid). log3 receives rows (shape, grid, median ms) of the last
- * sweep; returns its number of rows. The autotuner sweeps at the first run and once more after
- * 500 steps (on the state the run has reached), unless the cache answered. */
+ * 2 small, 3 mid, 4 big, 5 columns of cells), out[1] = persistent grid (0 default), out[2] = 1
+ * when the choice came from the process's cache of earlier sweeps (same pair kind, forces, types,
+ * exclusions, size, density, list range and cell grid). log3 receives rows (shape,
+ * grid, median ms) of the last sweep; returns its number of rows. The autotuner sweeps at the first
+ * run and once more after 500 steps (on the state the run has reached), unless the cache answered,
+ * and times the list build again where columns have become crowded. */
 int hm_sys_nlist_launch(const hm_system* s, int out[3], float* log3, unsigned int max_rows);
 /* Forget every launch shape the autotuner has cached in this process. */
 void hm_tune_cache_clear(void);

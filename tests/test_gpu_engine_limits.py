@@ -60,3 +60,17 @@ def test_overflow_replay_matches_oracle(hoomd, cmax, nmax):
     assert np.abs(gp - (rp + ri * L)).max() < 1e-6
     assert np.abs(snap.particles.velocity - rv).max() < 1e-5
     assert sim.timestep == 50
+
+
+def test_primed_graphs_outlive_a_longer_chunk(hoomd):
+    """A piece of ten steps up to the next sort, then one of 150 (more than the first room for Bussi draws):
+    both graphs are there afterwards, and the count is theirs."""
+    from hoomd_amd import _lib
+    pos, vel, L = lj_state(8)
+    sim, _ = make_sim(hoomd, pos, vel, L, thermostat=hoomd.md.methods.thermostats.Bussi(kT=1.2),
+                      sorter=(200, 32))
+    sim.run(0)
+    _lib.check(_lib.lib().hm_sys_set_chunk(sim._system, 150, 1))
+    _lib.check(_lib.lib().hm_sys_set_timestep(sim._system, 190))
+    assert _lib.lib().hm_sys_prime(sim._system, 160) == 2
+    assert _lib.lib().hm_sys_prime(sim._system, 160) == 0

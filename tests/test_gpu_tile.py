@@ -1,6 +1,6 @@
-"""The list build over columns of cells (csrc/tile.hip), entry for entry against the oracle's rows:
-sizes around its first one, ragged cell grids, few cells along an axis, empty and crowded regions,
-types, exclusions and rows that overflow."""
+"""The list-build driver where cells hold a few particles, entry for entry against the oracle's rows: ragged
+cell grids, few cells along an axis, empty and crowded regions, types, exclusions and rows that overflow. The
+driver builds by the cell form; the column form (csrc/tile.hip) is tested in test_gpu_columns.py."""
 
 import numpy as np
 import pytest
@@ -51,8 +51,8 @@ def test_rows_equal_oracle(H, N, L, rcut, buff):
     same_rows(nlist(pos, L, rcut, buff), O.nlist_binned(O.Box(*L), pos, rcut, buff, full=True))
 
 
-def test_crowded_columns_take_the_unstaged_path(H):
-    """All particles in half of the box: twice the mean density, more than the stage holds."""
+def test_crowded_half_of_the_box(H):
+    """All particles in half of the box: twice the mean density."""
     from gpu_helpers import nlist
     pos, L = box_fluid(33000, (66.0, 60.0, 62.0), 3)
     pos[:, 0] = pos[:, 0] / 2 + L[0] / 4
