@@ -1230,7 +1230,7 @@ struct hm_system
     }
 
     // bucket of systems that share launch shapes: pair kind, force kinds, types, exclusions,
-    // log2 N in half steps, density, list range and cells per axis (coarse)
+    // log2 N in half steps, density, list range, cells per axis (coarse) and whether columns apply
     std::string tune_key()
     {
         const double vol = hbox.L[0] * hbox.L[1] * hbox.L[2];
@@ -1238,10 +1238,11 @@ struct hm_system
         std::string forces_kinds;
         for (auto& f : forces)
             forces_kinds += char('0' + f.kind);
-        std::snprintf(buf, sizeof(buf), "k%d f%s t%u x%d n%ld r%ld l%ld c%u", pair_kind(),
+        std::snprintf(buf, sizeof(buf), "k%d f%s t%u x%d n%ld r%ld l%ld c%u%s", pair_kind(),
                       forces_kinds.c_str(), ntypes, (max_excl && exclude_bonds) ? 1 : 0,
                       std::lround(2.0 * std::log2((double)N)), std::lround(N / vol * 40.0),
-                      std::lround((rcut_max + r_buff) * 10.0), std::min(dim[0], 64u) / 8);
+                      std::lround((rcut_max + r_buff) * 10.0), std::min(dim[0], 64u) / 8,
+                      columns_apply() ? " columns" : "");
         return buf;
     }
 

@@ -488,7 +488,7 @@ int hm_sys_set_nlist_launch(hm_system* s, int shape, unsigned int grid);
 /* List-build launch chosen by the autotuner: out[0] = workgroup shape (0 default, 1 tiny,
  * 2 small, 3 mid, 4 big, 5 columns of cells), out[1] = persistent grid (0 default), out[2] = 1
  * when the choice came from the process's cache of earlier sweeps (same pair kind, forces, types,
- * exclusions, size, density, list range and cell grid). log3 receives rows (shape,
+ * exclusions, size, density, list range, cell grid and use of columns). log3 receives rows (shape,
  * grid, median ms) of the last sweep; returns its number of rows. The autotuner sweeps at the first
  * run and once more after 500 steps (on the state the run has reached), unless the cache answered,
  * and times the list build again where columns have become crowded. */

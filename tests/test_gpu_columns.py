@@ -291,3 +291,26 @@ def test_shape_set_by_the_caller_is_kept(hoomd):
     shape, cached, log = nlist_launch(sim)
     assert cached or shape == log[np.argmin(log[:, 2]), 0]
     assert _lib.lib().hm_sys_set_nlist_launch(sim._system, 6, 0) == -2
+
+
+def test_tuner_cache_keeps_the_forms_apart(hoomd):
+    """33 000 particles may be built over columns, 32 600 may not: the smaller system is swept by itself."""
+    from hoomd_amd import _lib
+    _lib.lib().hm_tune_cache_clear()
+    for N in (33000, 32600):
+        pos, L = lattice(33000, (32.0, 32.1, 32.2), 13)
+        keep = np.random.default_rng(1).permutation(33000)[:N]
+        snap = hoomd.Snapshot()
+        snap.configuration.box = [*L, 0, 0, 0]
+        snap.particles.N = N
+        snap.particles.types = ["A"]
+        snap.particles.position[:] = pos[keep]
+        sim = hoomd.Simulation(device=hoomd.device.GPU(), seed=1)
+        sim.create_state_from_snapshot(snap)
+        lj = hoomd.md.pair.LJ(nlist=hoomd.md.nlist.Cell(buffer=0.4), default_r_cut=WCA)
+        lj.params[("A", "A")] = dict(epsilon=1.0, sigma=1.0)
+        sim.operations.integrator = hoomd.md.Integrator(
+            dt=0.002, forces=[lj], methods=[hoomd.md.methods.ConstantVolume(hoomd.filter.All())])
+        sim.run(0)
+        shape, cached, log = nlist_launch(sim)
+        assert not cached and len(log) > 1 and (COLUMNS in log[:, 0]) == (N >= 32768)
