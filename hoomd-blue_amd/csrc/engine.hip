@@ -948,9 +948,11 @@ struct hm_system
         a2.finish = st;
     }
 
-    // room for the Bussi draws of a chunk of K steps (graphs hold its address)
-    void reserve_draws(unsigned int K)
+    // room for the Bussi draws of the longest chunk of a run: graphs hold its address, so it is made before
+    // the first of them is captured
+    void reserve_draws(uint64_t nsteps)
     {
+        const unsigned int K = (unsigned int)std::min<uint64_t>(chunk ? chunk : 1, nsteps);
         if (method != 1 || K <= n_draws)
             return;
         hchk(hipStreamSynchronize(stream), "sync");
@@ -1456,7 +1458,6 @@ struct hm_system
     // ------------------------------------------------------------------ run
     void launch_chunk(unsigned int K)
     {
-        reserve_draws(K);
         if (!use_graph)
         {
             launch_steps(K);
@@ -1499,6 +1500,7 @@ struct hm_system
             prep();
         if (!use_graph)
             return 0;
+        reserve_draws(nsteps);
         int added = 0;
         uint64_t t = timestep, end = timestep + nsteps;
         while (t < end)
@@ -1512,7 +1514,6 @@ struct hm_system
             const uint64_t ran = steps_run + (t - timestep);
             if (autotune && !retuned && !tune_cached && ran < retune_after)
                 K = std::min<uint64_t>(K, retune_after - ran);
-            reserve_draws((unsigned int)K);
             if (graphs.find((unsigned int)K) == graphs.end())
             {
                 graphs.emplace((unsigned int)K, capture_steps((unsigned int)K));
@@ -1539,6 +1540,7 @@ struct hm_system
         }
         if (!prepared)
             prep();
+        reserve_draws(nsteps);
         uint64_t end = timestep + nsteps;
         int retries = 0;
         while (timestep < end)
