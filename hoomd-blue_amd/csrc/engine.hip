@@ -1097,18 +1097,29 @@ struct hm_system
     }
 
     // Autotuner (the role of Autotuner.h): every candidate launch configuration of the pair
-    // kernel in use is timed over 5 launches with HIP events on the engine stream, and the one
+    // kernel in use is timed over 5 samples with HIP events on the engine stream, and the one
     // with the smallest median launch time is kept -- the reference's protocol of sampling each
     // parameter tuple 5 times and taking the median (Autotuner.h:503-664). Candidates: lanes per
     // particle {1, 2, 4, 8, 16} x block size {64, 128, 256, 512, 1024} for the gather kernels,
     // lanes per particle {4, 8, 16} for the cell-tiled kernel. The pair launches only rewrite
     // the force arrays with the same values, so tuning does not change the state.
-    // Sweep of the list build's workgroup shape and persistent grid on the lists of the current
-    // state (cells already built; every candidate writes the same rows), median of 3 launches.
-    // Launches per timed sample. A single launch of a few microseconds between two events reads the
-    // event and dispatch time, not the kernel's: at 2 048 particles the sweep kept one lane per particle
-    // (7.8 us a launch) where eight take 4.0.
-    unsigned int tune_repeat() const { return N <= 262144 ? 16u : 1u; }
+    // Launches per timed sample of a candidate: about 40 us of them, so that the event and dispatch time of
+    // a few microseconds does not decide between launches of the same length (at 2 048 particles single
+    // launches kept one lane per particle, 7.8 us a launch where eight take 3.7), and no more, because a
+    // program waits for the sweep at its first run: 13 ms for 2 048 LJ particles, 32 for 131 072 and 61 for
+    // 262 144, where 16 launches a sample took 42, 237 and 560 and chose the same, and one takes 6, 24, 51.
+    static constexpr float TUNE_SAMPLE_MS = 0.04f;
+    template<class F> unsigned int sample_launches(F&& launch, hipEvent_t e0, hipEvent_t e1)
+    {
+        launch();  // code and caches
+        hchk(hipEventRecord(e0, stream), "event");
+        launch();
+        hchk(hipEventRecord(e1, stream), "event");
+        hchk(hipEventSynchronize(e1), "event");
+        float t = 0.f;
+        hchk(hipEventElapsedTime(&t, e0, e1), "event");
+        return (unsigned int)std::min(16.0f, std::max(1.0f, std::ceil(TUNE_SAMPLE_MS / std::max(t, 1e-4f))));
+    }
     struct NlSample
     {
         int shape;
@@ -1116,6 +1127,8 @@ struct hm_system
         float ms;
     };
     std::vector<NlSample> nl_log;
+    // Sweep of the list build's workgroup shape and persistent grid on the lists of the current
+    // state (cells already built; every candidate writes the same rows), median of 3 samples.
     void tune_nlist()
     {
         nl_log.clear();
@@ -1155,12 +1168,13 @@ struct hm_system
                 NlistKernelArgs k;
                 fill_nlist_args(k, false);
                 k.counter = nullptr;
-                hchk(launch_nlist_build(k, stream), "nlist tune");
+                auto build = [&]() { hchk(launch_nlist_build(k, stream), "nlist tune"); };
+                const unsigned int n = sample_launches(build, ev[0], ev[1]);
                 for (int r = 0; r < 3; r++)
                 {
                     hchk(hipEventRecord(ev[r], stream), "event");
-                    for (unsigned int q = 0; q < tune_repeat(); q++)
-                        hchk(launch_nlist_build(k, stream), "nlist tune");
+                    for (unsigned int q = 0; q < n; q++)
+                        build();
                 }
                 hchk(hipEventRecord(ev[3], stream), "event");
                 hchk(hipEventSynchronize(ev[3]), "event");
@@ -1168,7 +1182,7 @@ struct hm_system
                 for (int r = 0; r < 3; r++)
                     hchk(hipEventElapsedTime(&t[r], ev[r], ev[r + 1]), "event");
                 std::sort(t, t + 3);
-                t[1] /= (float)tune_repeat();
+                t[1] /= (float)n;
                 nl_log.push_back({sh, g, t[1]});
                 if (t[1] < best)
                 {
@@ -1286,12 +1300,13 @@ struct hm_system
         for (const PairLaunch& c : cands)
         {
             cfg = c;
-            launch_pair(*f, compute_virial);  // warm-up launch
+            auto pair = [&]() { launch_pair(*f, compute_virial); };
+            const unsigned int n = sample_launches(pair, ev[0], ev[1]);
             for (int r = 0; r < 5; r++)
             {
                 hchk(hipEventRecord(ev[r], stream), "event");
-                for (unsigned int q = 0; q < tune_repeat(); q++)
-                    launch_pair(*f, compute_virial);
+                for (unsigned int q = 0; q < n; q++)
+                    pair();
             }
             hchk(hipEventRecord(ev[5], stream), "event");
             hchk(hipEventSynchronize(ev[5]), "event");
@@ -1299,7 +1314,7 @@ struct hm_system
             for (int r = 0; r < 5; r++)
                 hchk(hipEventElapsedTime(&t[r], ev[r], r < 4 ? ev[r + 1] : ev[5]), "event");
             std::sort(t, t + 5);
-            t[2] /= (float)tune_repeat();
+            t[2] /= (float)n;
             tune_log.push_back({c.tpp, c.block, c.batch, t[2]});
             if (t[2] < best)
             {

@@ -471,7 +471,7 @@ int hm_sys_set_pair_launch(hm_system* s, unsigned int tpp, unsigned int block_si
 int hm_sys_set_pair_kernel(hm_system* s, int kind, unsigned int tpp, unsigned int size);
 /* Autotuner (replaces Autotuner.h, hoomd/Autotuner.h:503-664): when on (the default, and after
  * hm_sys_set_pair_kernel with tpp = size = 0) the next run first times every launch
- * configuration of the pair kernel in use (5 launches each, median) and keeps the fastest.
+ * configuration of the pair kernel in use (5 samples each, median) and keeps the fastest.
  * An explicit tpp / block size turns it off. */
 int hm_sys_set_autotune(hm_system* s, int on);
 /* Pair launch in use: out[0] = kind actually run, out[1] = tpp, out[2] = block size (kind 1, 2)

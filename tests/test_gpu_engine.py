@@ -371,6 +371,32 @@ def test_autotuner_sweeps_and_keeps_results(hoomd):
     assert rows == 0 and nl[2] == 1 and sim.operations.is_tuning_complete
 
 
+def test_sweep_is_a_short_part_of_the_first_run(hoomd):
+    """A candidate is launched twice and then sampled (5 times for the pair kernel, 3 for the list) over about
+    40 us or one launch. Twice that time, and 30 ms for the host, hold the sweep of 131 072 particles."""
+    import time
+    from hoomd_amd import _lib
+    from lattices import perturbed_fcc
+    pos, L = perturbed_fcc(32, 0.8442, r=0.05, seed=1)
+    _lib.lib().hm_tune_cache_clear()
+    took = []
+    for swept in (True, False):
+        sim, lj = make_sim(hoomd, pos, np.zeros_like(pos), L)
+        t0 = time.perf_counter()
+        sim.run(0)
+        took.append(time.perf_counter() - t0)
+        if swept:
+            tl, nl = np.zeros((64, 4), np.float32), np.zeros((64, 3), np.float32)
+            a = _lib.lib().hm_sys_tune_log(sim._system, tl.ctypes.data, 64)
+            b = _lib.lib().hm_sys_nlist_launch(sim._system, np.zeros(3, np.int32).ctypes.data, nl.ctypes.data, 64)
+            assert a > 0 and b > 0
+            work = 1e-3 * sum((2 * t + n * np.maximum(t, 0.04) + n * t).sum()
+                              for n, t in ((5, tl[:a, 3]), (3, nl[:b, 2])))
+    print(f"first run {took[0] * 1e3:.1f} ms swept, {took[1] * 1e3:.1f} ms from the cache, sweep's launches "
+          f"{work * 1e3:.1f} ms", flush=True)
+    assert took[0] - took[1] < 2 * work + 0.03
+
+
 @pytest.mark.parametrize("delay,dist,kT", [(3, False, 1.2), (0, False, 1.2), (4, True, 40.0),
                                            (1, True, 40.0)])
 def test_rebuild_policy_matches_oracle(hoomd, delay, dist, kT):
