@@ -2279,6 +2279,7 @@ int hm_sys_set_state(hm_system* s, const double* pos3, const double* vel3, const
         hchk(hipMemcpy(s->vel, v.data(), sizeof(double4) * N, hipMemcpyHostToDevice), "upload");
         hchk(hipMemcpy(s->image, im.data(), sizeof(i3) * N, hipMemcpyHostToDevice), "upload");
         s->prepared = false;
+        s->configured = false;  // a training call checks the positions it was given, as a run does
         return HM_OK;
     });
 }
