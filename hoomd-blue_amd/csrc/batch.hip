@@ -95,7 +95,6 @@ struct Rep
 constexpr unsigned int REL_MIN_DIM = 4;
 constexpr unsigned int BCODE_SHIFT = 26;
 constexpr unsigned int BJ_MASK = (1u << BCODE_SHIFT) - 1u;
-constexpr unsigned int BCODE_SELF = 13u; // offset (0, 0, 0)
 
 // per-replica device state
 struct RepState

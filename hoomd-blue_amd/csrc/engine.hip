@@ -1105,7 +1105,7 @@ struct hm_system
     // the force arrays with the same values, so tuning does not change the state.
     // Launches per timed sample of a candidate: about 40 us of them, so that the event and dispatch time of
     // a few microseconds does not decide between launches of the same length (at 2 048 particles single
-    // launches kept one lane per particle, 7.8 us a launch where eight take 3.7), and no more, because a
+    // launches kept one lane per particle, 7.8 us a launch where eight take 4.0), and no more, because a
     // program waits for the sweep at its first run: 13 ms for 2 048 LJ particles, 32 for 131 072 and 61 for
     // 262 144, where 16 launches a sample took 42, 237 and 560 and chose the same, and one takes 6, 24, 51.
     static constexpr float TUNE_SAMPLE_MS = 0.04f;

@@ -55,8 +55,9 @@ __device__ __forceinline__ int sorted_neighbour(int h, int d, int k, int& n)
     return off;
 }
 
-// Minimum-image offset of a position from a cell centre, rounded to FP32 (dims >= 4 keeps every
-// staged particle within 1.5 cell widths of the centre, well inside half a box).
+// Minimum-image offset of a position from a centre, rounded to FP32. The caller keeps every staged particle
+// inside half a box of it: within 1.5 cell widths of a cell's centre on grids of 4 cells or more, within
+// half a column and one layer of a column's (up to 9 cell widths; choose_columns).
 __device__ __forceinline__ float3 rel_to_centre(const DevBox& b, double x, double y, double z,
                                                 double cx, double cy, double cz)
 {

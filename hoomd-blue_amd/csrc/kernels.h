@@ -483,8 +483,10 @@ struct StepMidArgs
     double ndof, tau, kT;    // Bussi
     const BussiDraws* draws; // of the step that begins
 };
-// Adding up to 1 024 partials (8 KB) in every workgroup costs less than the launch it saves (the step at
-// 131 072 particles fell from 37.7 to 33.8 us with it and the fused launch); 4 096 would be 134 MB.
+// Adding up to 1 024 partials (8 KB) in every workgroup costs less than the launch it saves. Every workgroup
+// adding -> one workgroup in a launch of its own, us a step of a WCA fluid, 128 partials 21.5 -> 22.4, 512 35.1
+// -> 36.3, 1 024 54.3 -> 56.1, 2 048 between -2 and +3 % from run to run, 4 096 203 -> 200: past 1 024 the
+// partials grow with the square of the particles and nothing is left to win.
 constexpr unsigned int MID_SUM_MAX_PARTIAL = 1024;
 hipError_t launch_step_mid(const StepMidArgs& a, hipStream_t s);
 // Kinetic-energy partials of the velocities after step two (which are not stored)

@@ -971,14 +971,14 @@ static void nlist_dispatch(const NlistKernelArgs& a, bool mt, bool ex, unsigned 
 }
 
 // Where cells hold a few particles the list can be built over columns (tile.hip). Index rows, us a build,
-// cell form below -> columns: 10^6 particles, 3.0 a cell 405 -> 254, 6.7 a cell 397 -> 302; 131 072, 3.1 a
-// cell 58 -> 38, 7.5 a cell 59 -> 43; 50 021, 3.2 a cell 27 -> 22, 7.3 a cell 28 -> 24; at 16 384 the two are
-// equal (15 -> 16), and at 21 a cell the cell form's wavefront per home particle is the better one (520
-// against 606 at 10^6). These are uniform fluids. A slab of 20 a cell beside vapour (33 000 particles, 6.7 on
-// the mean) takes 248 us over columns and 37 in the cell form, which the mean does not tell: columns are
-// built only where the caller asks for them, as the engine does after timing both. The cell form also keeps
-// the 16-bit local rows, grids with fewer than 4 cells along an axis, and exclusions given without the slot
-// of each particle.
+// best shape of the cell form -> columns: 10^6 particles, 3.6 a cell 355 -> 269, 7.1 a cell 323 -> 239;
+// 131 072, 3.6 a cell 54 -> 40, 7.5 a cell 54 -> 43; 50 021, 25 -> 23 and 27 -> 23; 33 000, 21 -> 20 and
+// 24 -> 23; at 16 384 the two are equal, and at 21 a cell the cell form's wavefront per home particle is the
+// better one (520 against 606 at 10^6). These are uniform fluids. A slab of 20 a cell beside vapour (33 000
+// particles, 6.7 on the mean) takes 249 us over columns and 37 in the cell form, which the mean does not
+// tell: columns are built only where the caller asks for them, as the engine does after timing both. The
+// cell form also keeps the 16-bit local rows, grids with fewer than 4 cells along an axis, and exclusions
+// given without the slot of each particle.
 constexpr unsigned int COL_MIN_N = 32768;
 
 static bool column_build_applies(const NlistKernelArgs& a, ColGeom& g)

@@ -11,7 +11,6 @@ namespace hm
 
 constexpr unsigned int COL_BLOCK = 256;
 constexpr unsigned int COL_PAD = 32;         // readable entries after the staged particles
-constexpr unsigned int COL_MAX_CAP = 3072;  // staged particles: 48 KB
 
 bool choose_columns(unsigned int N, const unsigned int dim[3], ColGeom& g)
 {
@@ -28,7 +27,7 @@ bool choose_columns(unsigned int N, const unsigned int dim[3], ColGeom& g)
     g.ntile = dim[0] * dim[1] * g.nz;
     const double st = mean * 9.0 * (tallest + 2.0);
     const double cap = st * 1.25 + 4.0 * std::sqrt(st) + 64.0;
-    g.cap = (unsigned int)std::min((double)COL_MAX_CAP, std::ceil(cap / 64.0) * 64.0);
+    g.cap = (unsigned int)(std::ceil(cap / 64.0) * 64.0);  // at most 1 728 at 8 a cell: 28 KB
     g.hcap = g.cap / 4;
     g.lpc = 4;
     while (g.lpc < 32 && g.lpc < mean * 1.2)
@@ -155,10 +154,12 @@ struct ColHome
 // entries are cell slots with offset codes in transposed blocks (pair_rel_kernel's rows), else
 // particle indices.
 //
-// The one-wavefront-per-cell form this replaces staged 27 cells for every home cell of about three
-// particles and compacted every 64 tests by ballot (about 765 vector instructions per cell). At
-// 10^6 particles, 3.0 per cell, 12.5 neighbours: 254 us a build, before 405. What bounds it now is the
-// chain of each column (cell sizes, staging, rows) with eight workgroups per CU in flight.
+// The one-wavefront-per-cell form stages 27 cells for every home cell of about three particles and compacts
+// every 64 tests by ballot (about 765 vector instructions per cell). 10^6 beads of a melt, 3.0 a cell, 12.5
+// neighbours, exclusions: 370 us a build, that form 553. Waves wait 70 % of their cycles (SQ_WAIT_ANY 619 M
+// of 882 M); the 200 MB it reads and 135 MB it writes would take 70 us, its 114 M vector instructions 190
+// (four cycles each on 1 024 SIMDs): what bounds it is the chain of each column (cell sizes, staging, rows)
+// with five to seven workgroups per CU in flight.
 template<int G, bool MT, bool EXCL, bool SLOT>
 __global__ __launch_bounds__(COL_BLOCK) void nlist_col_kernel(NlistKernelArgs a, ColGeom g)
 {
