@@ -507,7 +507,7 @@ __global__ __launch_bounds__(64 * NL_WAVES) void bnlist_kernel(
                 const uint64_t m = wave_ballot(hit);
                 const unsigned int at = cnt + lanes_below(m);
                 if (hit && at < nmax)
-                    row[row_store_pos(at)] = e;
+                    row[rel ? row_store_pos(at) : at] = e;
                 cnt += (unsigned int)__popcll(m);
             }
             if (lane == 0)
@@ -543,9 +543,11 @@ __device__ __forceinline__ void lj_accumulate(const PairConst& pc, float rsq, fl
     fz += dz * fdr;
 }
 
-// Rows are in transposed blocks of ROW_BLOCK entries (row_store_pos): a lane reads four entries with one
-// 16-byte load, and for each of the four the lanes of a particle hold consecutive neighbours. The cell
-// offset of an entry comes from a table in LDS. Workgroups are in XCD order, so a replica's particles
+// Rows of boxes with relative positions are in transposed blocks of ROW_BLOCK entries (row_store_pos): a lane
+// reads four entries with one 16-byte load, and for each of the four the lanes of a particle hold
+// consecutive neighbours. Smaller boxes (FP64) keep the rows as they are and 4-byte loads, whose lanes are
+// adjacent: in blocks a launch of 256 replicas of 1 000 took 71 us where this takes 58 (1 024 of 250: 70, 56).
+// The cell offset of an entry comes from a table in LDS. Workgroups are in XCD order, so a replica's particles
 // stay in one L2. 1.3e6 particles in 256 replicas, 105e6 entries: 210 us a launch, before 218 (4-byte row
 // loads, the offset decoded by divisions: 25 vector instructions of a pair's 60).
 template<unsigned int TPP>
@@ -628,7 +630,7 @@ __global__ __launch_bounds__(256) void bpair_kernel(
             for (unsigned int u = 0; u < UNR; u++)
             {
                 const unsigned int k = k0 + u * TPP;
-                j[u] = k < nn ? row[row_store_pos(k)] : p;
+                j[u] = k < nn ? row[k] : p;
             }
             double4 xj[UNR];
 #pragma unroll
